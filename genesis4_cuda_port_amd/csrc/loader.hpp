@@ -54,14 +54,19 @@ __host__ __device__ inline double normal(uint64_t stream, uint64_t k) {
 // Phi(x) = erfc(-x/sqrt2)/2, started from the Tukey-lambda approximation
 // x0 = 4.91 (p^0.14 - (1-p)^0.14).  The upper half uses Phi^-1(p) =
 // -Phi^-1(1-p) (1-p is exact there) so both tails are solved where erfc is
-// accurate.
+// accurate.  The start is within 1e-2 (its powers need only FP32) and a step
+// of size d leaves an error of (2x^2+1)/6 d^3 < 1e-16 for d <= 1e-6, so the
+// iteration ends there: two steps for 99 % of p.  Waiting for a step of 1e-16
+// instead ran to the limit wherever the rounding of Phi(x) - p exceeds it (one
+// p in nine, so every wave): generating 4096 x 16384 particles took 29.2 ms.
 __host__ __device__ inline double inverse_normal(double p) {
   double sign = 1.0;
   if (p > 0.5) {
     p = 1.0 - p;
     sign = -1.0;
   }
-  double x = 4.91 * (pow(p, 0.14) - pow(1.0 - p, 0.14));
+  const float pf = static_cast<float>(p), qf = static_cast<float>(1.0 - p);
+  double x = 4.91 * (static_cast<double>(powf(pf, 0.14f)) - static_cast<double>(powf(qf, 0.14f)));
   for (int it = 0; it < 60; ++it) {
     const double phi = 0.5 * erfc(-x / sqrt(2.0));
     const double pdf = exp(-0.5 * x * x) / sqrt(2.0 * kPi);
@@ -70,7 +75,7 @@ __host__ __device__ inline double inverse_normal(double p) {
     const double r = f / pdf;
     const double dx = r / (1.0 + 0.5 * x * r);
     x -= dx;
-    if (fabs(dx) <= 1e-16 * fmax(1.0, fabs(x))) break;
+    if (fabs(dx) <= 1e-6) break;
   }
   return sign * x;
 }
