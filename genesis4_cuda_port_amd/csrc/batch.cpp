@@ -17,7 +17,7 @@
 // EVERY run as one launch per kernel on the batch's stream (G4H_TUNE_BATCH =
 // 0, the default): the particle passes (one workgroup per run, its group's
 // beam slice and parameter entry), the x and the y sweep (one workgroup per
-// 64-line block of every run's plane, its group's tables of the step), and on
+// 16-line block of every run's plane, its group's tables of the step), and on
 // output steps one kernel writing every run's field record.  Three or four
 // launches per step, whatever the number of grids: per-group launches on
 // per-group streams (G4H_TUNE_BATCH = 2, and what other batches run) spent
@@ -233,7 +233,7 @@ struct g4h_batch {
 
   // The per-step launches of every run: run descriptors as for the one-launch
   // path, plus each run's x-sweep output and partials, and one descriptor per
-  // 64-line block of every plane.  Returns false (the batch keeps the
+  // 16-line block of every plane.  Returns false (the batch keeps the
   // per-group launches) for grids above the segmented sweeps' limit or when
   // the source is on in some groups and off in others at some step.
   bool setup_grid(Context* c) {
@@ -303,7 +303,7 @@ struct g4h_batch {
       Group& g = groups[gi];
       Field* f = g.field;
       const int n = static_cast<int>(g.runs.size());
-      const int nblk = (g.G + 63) / 64;
+      const int nblk = (g.G + kAdiSegLines - 1) / kAdiSegLines;
       for (int i = 0; i < n; ++i)
         for (int b = 0; b < nblk; ++b) {
           BatchSegDesc d{};
@@ -355,7 +355,7 @@ struct g4h_batch {
       if (f->adi_y.size() < static_cast<size_t>(f->cells())) f->adi_y.alloc(f->ctx, f->cells());
       ensure_source(f);
       (void)field_adi_ustar(f);
-      const int nblk = (g.G + 63) / 64;
+      const int nblk = (g.G + kAdiSegLines - 1) / kAdiSegLines;
       const size_t need = g.runs.size() * static_cast<size_t>(nblk) * 8 + 2 * g.runs.size();
       if (f->col_partials.size() < need) f->col_partials.alloc(f->ctx, need);
       dadi[gi].alloc(g.gctx, static_cast<size_t>(ns));

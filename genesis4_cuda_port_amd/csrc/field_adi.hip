@@ -19,7 +19,7 @@
 //    plane when asked.
 // The RHS, the source add and the Thomas recurrences are FP64 in both
 // precisions; the stored field is FP32 in MIXED.
-#include "adi_lines.hpp"
+#include "adi_seg.hpp"
 
 #include <complex>
 #include <vector>
@@ -364,80 +364,97 @@ __global__ __launch_bounds__(kLane) void adi_y_lane_kernel(typename A2<P>::T* u,
   }
 }
 
-// Segmented sweeps (adi_lines.hpp): a workgroup of kSegs waves per 64 lines
-// of a plane, every element in registers between its load and its store,
-// the tables of the step (c, cbet, cwet, beta, delta) staged in LDS.  For
-// G <= kSegs * kSegMax.
-template <class P, int LPW>
-__global__ __launch_bounds__(adi::kSegs * LPW, 4) void adi_x_seg_kernel(
-    const typename A2<P>::T* u, typename A2<P>::T* ustar, int nslice, int G, int m, double cs,
+// Segmented sweeps (adi_seg.hpp), for G <= 256.  Workgroups go to the XCDs
+// round robin, so block b takes line block (b / 8) % nblk of a plane of the
+// planes b % 8, b % 8 + 8, ...: the blocks of a plane, which share rows and
+// the cache lines that their row segments cut, run on one XCD and its L2.
+// Bound: HBM.  Before, a workgroup of 16 waves took 64 lines, one lane per
+// row in the x sweep (64 cache lines per load) and one workgroup per CU.
+//                                        x sweep            y sweep
+//   2048 planes, G = 255, MIXED      1528 ->  428 us     871 -> 467 us
+//   1024 planes, G = 151, FP64        333 ->  152 us     293 -> 160 us
+//   1 plane, G = 151, FP64           20.5 ->  5.3 us    20.1 -> 5.4 us
+//   batch of 96 planes, MIXED          51 ->   21 us      37 ->  26 us
+// (2.13 and 0.75 GB read and written: 5.0 / 4.6 and 4.9 / 4.7 TB/s; the card
+// scales 2 GiB in place at 5.95 TB/s).  The y sweep with nontemporal accesses
+// took 883 and 235 us: its row segments cut cache lines that the next
+// block's complete in L2.  Both sweeps launched plane chunk by plane chunk,
+// so that the intermediate planes stay in the 256 MB last-level cache,
+// gained nothing at 64-256 MB per chunk and lost below.
+struct SegBlock {
+  int p, blk;
+};
+__device__ __forceinline__ SegBlock seg_block(int nblk) {
+  const int b = blockIdx.x, i = b >> 3;
+  return SegBlock{(i / nblk) * 8 + (b & 7), i % nblk};
+}
+
+template <class P, int K>
+__global__ __launch_bounds__(adi::kSegThreads, K > 10 ? 3 : 4) void adi_x_seg_kernel(
+    const typename A2<P>::T* u, typename A2<P>::T* ustar, int nslice, int nblk, int G, double cs,
     const double2* __restrict__ tab, const typename A2<P>::T* src, const int4* rect, int first,
     int add_src) {
   using T2 = typename A2<P>::T;
   extern __shared__ double2 lds[];
-  for (int k = threadIdx.x; k < 5 * G; k += blockDim.x) lds[k] = tab[k];
+  const SegBlock b = seg_block(nblk);
+  if (b.p >= nslice) return;
+  for (int k = threadIdx.x; k < adi::seg_table_size(K); k += blockDim.x) lds[k] = tab[k];
   __syncthreads();
-  const int p = blockIdx.x;
   const int64_t plane = static_cast<int64_t>(G) * G;
-  const int s = ((p - first) % nslice + nslice) % nslice;
+  const int s = ((b.p - first) % nslice + nslice) % nslice;
   int4 rc = make_int4(0, 0, 0, 0);
   const T2* sp = nullptr;
   if (add_src) {
     rc = rect[s];
     sp = src + s * plane;
   }
-  const adi::SegTables tb{lds, lds + G, lds + 2 * G, lds + 3 * G, lds + 4 * G};
-  adi::seg_sweep<P, LPW, true, false>(u + p * plane, ustar + p * plane, G, m, cs, tb, sp, rc,
-                                 blockIdx.y, lds + 5 * G, nullptr, nullptr, nullptr);
+  adi::seg_x<P, K>(u + b.p * plane, ustar + b.p * plane, G, cs, lds, sp, rc, b.blk,
+                   reinterpret_cast<double*>(lds + adi::seg_table_size(K)));
 }
 
 // ... and the y sweep, with the block's field sums in the layout of the
 // wave-per-block variants (partials[(p * nblk + b) * 8 + k], centres at the
 // tail).
-template <class P, int LPW>
-__global__ __launch_bounds__(adi::kSegs * LPW, 4) void adi_y_seg_kernel(
-    typename A2<P>::T* u, const typename A2<P>::T* ustar, int nslice, int G, int m, double cs,
+template <class P, int K, bool STATS>
+__global__ __launch_bounds__(adi::kSegThreads, K > 10 ? 3 : 4) void adi_y_seg_kernel(
+    typename A2<P>::T* u, const typename A2<P>::T* ustar, int nslice, int nblk, int G, double cs,
     const double2* __restrict__ tab, const typename A2<P>::T* src, const int4* rect, int first,
     int add_src, double* partials) {
   using T2 = typename A2<P>::T;
   extern __shared__ double2 lds[];
-  __shared__ double red[adi::kSegs * LPW / kLane * 8];
-  for (int k = threadIdx.x; k < 5 * G; k += blockDim.x) lds[k] = tab[k];
+  const SegBlock b = seg_block(nblk);
+  if (b.p >= nslice) return;
+  for (int k = threadIdx.x; k < adi::seg_table_size(K); k += blockDim.x) lds[k] = tab[k];
   __syncthreads();
-  const int p = blockIdx.x;
-  const int nblk = gridDim.y;
   const int64_t plane = static_cast<int64_t>(G) * G;
-  const int s = ((p - first) % nslice + nslice) % nslice;
+  const int s = ((b.p - first) % nslice + nslice) % nslice;
   int4 rc = make_int4(0, 0, 0, 0);
   const T2* sp = nullptr;
   if (add_src) {
     rc = rect[s];
     sp = src + s * plane;
   }
-  const adi::SegTables tb{lds, lds + G, lds + 2 * G, lds + 3 * G, lds + 4 * G};
-  if (partials) {
-    double* part = partials + (static_cast<int64_t>(p) * nblk + blockIdx.y) * 8;
-    double* centre = partials + static_cast<int64_t>(nslice) * nblk * 8 + 2 * p;
-    adi::seg_sweep<P, LPW, false, true>(ustar + p * plane, u + p * plane, G, m, cs, tb, sp, rc,
-                                   blockIdx.y, lds + 5 * G, red, part, centre);
-  } else {
-    adi::seg_sweep<P, LPW, false, false>(ustar + p * plane, u + p * plane, G, m, cs, tb, sp, rc,
-                                    blockIdx.y, lds + 5 * G, nullptr, nullptr, nullptr);
-  }
+  double2* ends = lds + adi::seg_table_size(K);
+  double* red = reinterpret_cast<double*>(ends + 2 * adi::kSegs * adi::kSegLines);
+  double* part = STATS ? partials + (static_cast<int64_t>(b.p) * nblk + b.blk) * 8 : nullptr;
+  double* centre = STATS ? partials + static_cast<int64_t>(nslice) * nblk * 8 + 2 * b.p : nullptr;
+  adi::seg_y<P, K, STATS>(ustar + b.p * plane, u + b.p * plane, G, cs, lds, sp, rc, b.blk, ends,
+                          red, part, centre, nullptr);
 }
 
 // The segmented sweeps of every run of a batch in one launch: workgroup b
-// takes block b of the descriptor list (one run's 64-line block), the run's
+// takes block b of the descriptor list (one run's 16-line block), the run's
 // group tables and coefficient of step k.
 template <class P>
-__global__ __launch_bounds__(adi::kSegs * kLane, 4) void adi_x_seg_batch_kernel(
+__global__ __launch_bounds__(adi::kSegThreads, 3) void adi_x_seg_batch_kernel(
     const BatchSegDesc* __restrict__ blocks, int k, int add_src) {
   using T2 = typename A2<P>::T;
   extern __shared__ double2 lds[];
   const BatchSegDesc D = blocks[blockIdx.x];
   const int G = D.G;
-  const double2* tab = D.adi[k];
-  for (int i = threadIdx.x; i < 5 * G; i += blockDim.x) lds[i] = tab[i];
+  const double2* tab = D.adi[k] + 3 * G;
+  const int ntab = adi::seg_table_size(adi::seg_len(G));
+  for (int i = threadIdx.x; i < ntab; i += blockDim.x) lds[i] = tab[i];
   __syncthreads();
   const int64_t plane = static_cast<int64_t>(G) * G;
   int4 rc = make_int4(0, 0, 0, 0);
@@ -446,23 +463,25 @@ __global__ __launch_bounds__(adi::kSegs * kLane, 4) void adi_x_seg_batch_kernel(
     rc = D.rect[D.slice];
     sp = static_cast<const T2*>(D.src) + D.slice * plane;
   }
-  const adi::SegTables tb{lds, lds + G, lds + 2 * G, lds + 3 * G, lds + 4 * G};
-  adi::seg_sweep<P, kLane, true, false>(static_cast<const T2*>(D.u) + D.slice * plane,
-                                        static_cast<T2*>(D.ustar) + D.slice * plane, G,
-                                        (G + adi::kSegs - 1) / adi::kSegs, D.cs[k], tb, sp, rc,
-                                        D.blk, lds + 5 * G, nullptr, nullptr, nullptr);
+  const T2* in = static_cast<const T2*>(D.u) + D.slice * plane;
+  T2* out = static_cast<T2*>(D.ustar) + D.slice * plane;
+  const double cs = D.cs[k];
+  adi::with_seg_len(G, [&](auto len) {
+    adi::seg_x<P, decltype(len)::value>(in, out, G, cs, lds, sp, rc, D.blk,
+                                        reinterpret_cast<double*>(lds + ntab));
+  });
 }
 
 template <class P, bool STATS>
-__global__ __launch_bounds__(adi::kSegs * kLane, 4) void adi_y_seg_batch_kernel(
+__global__ __launch_bounds__(adi::kSegThreads, 3) void adi_y_seg_batch_kernel(
     const BatchSegDesc* __restrict__ blocks, int k, int add_src, int clear_src) {
   using T2 = typename A2<P>::T;
   extern __shared__ double2 lds[];
-  __shared__ double red[adi::kSegs * 8];
   const BatchSegDesc D = blocks[blockIdx.x];
   const int G = D.G;
-  const double2* tab = D.adi[k];
-  for (int i = threadIdx.x; i < 5 * G; i += blockDim.x) lds[i] = tab[i];
+  const double2* tab = D.adi[k] + 3 * G;
+  const int ntab = adi::seg_table_size(adi::seg_len(G));
+  for (int i = threadIdx.x; i < ntab; i += blockDim.x) lds[i] = tab[i];
   __syncthreads();
   const int64_t plane = static_cast<int64_t>(G) * G;
   int4 rc = make_int4(0, 0, 0, 0);
@@ -471,20 +490,20 @@ __global__ __launch_bounds__(adi::kSegs * kLane, 4) void adi_y_seg_batch_kernel(
     rc = D.rect[D.slice];
     sp = static_cast<const T2*>(D.src) + D.slice * plane;
   }
-  const adi::SegTables tb{lds, lds + G, lds + 2 * G, lds + 3 * G, lds + 4 * G};
-  const int m = (G + adi::kSegs - 1) / adi::kSegs;
   const T2* in = static_cast<const T2*>(D.ustar) + D.slice * plane;
   T2* out = static_cast<T2*>(D.u) + D.slice * plane;
   T2* clr = clear_src && sp ? const_cast<T2*>(sp) : nullptr;
-  if constexpr (STATS) {
-    double* part = D.partials + (static_cast<int64_t>(D.slice) * D.nblk + D.blk) * 8;
-    double* centre = D.partials + static_cast<int64_t>(D.nrun) * D.nblk * 8 + 2 * D.slice;
-    adi::seg_sweep<P, kLane, false, true>(in, out, G, m, D.cs[k], tb, sp, rc, D.blk,
-                                          lds + 5 * G, red, part, centre, clr);
-  } else {
-    adi::seg_sweep<P, kLane, false, false>(in, out, G, m, D.cs[k], tb, sp, rc, D.blk,
-                                           lds + 5 * G, nullptr, nullptr, nullptr, clr);
-  }
+  double2* ends = lds + ntab;
+  double* red = reinterpret_cast<double*>(ends + 2 * adi::kSegs * adi::kSegLines);
+  double* part =
+      STATS ? D.partials + (static_cast<int64_t>(D.slice) * D.nblk + D.blk) * 8 : nullptr;
+  double* centre =
+      STATS ? D.partials + static_cast<int64_t>(D.nrun) * D.nblk * 8 + 2 * D.slice : nullptr;
+  const double cs = D.cs[k];
+  adi::with_seg_len(G, [&](auto len) {
+    adi::seg_y<P, decltype(len)::value, STATS>(in, out, G, cs, lds, sp, rc, D.blk, ends, red, part,
+                                               centre, clr);
+  });
 }
 
 // Field record r of every run from its block partials, summed in block order
@@ -494,7 +513,7 @@ __global__ void batch_field_record_kernel(const BatchRunDesc* __restrict__ runs,
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nruns) return;
   const BatchRunDesc R = runs[i];
-  const int nblk = (R.G + kLane - 1) / kLane;
+  const int nblk = (R.G + adi::kSegLines - 1) / adi::kSegLines;
   double* o = R.field_hist + (static_cast<int64_t>(r) * R.nrun + R.slice) * G4H_FIELD_RAW;
   for (int q = 0; q < 7; ++q) {
     double v = 0.0;
@@ -537,42 +556,44 @@ void adi_step(Field* f, bool source_on, bool stats) {
   // registers).  Tuned per shape; all three give bit-identical fields.
   //
   // Variant 3, the segmented sweeps, holds every element in registers (no
-  // FP64 forward-value plane) and spreads a line over kSegs waves; it rounds
+  // FP64 forward-value plane) and spreads a line over 16 lanes; it rounds
   // differently from the single-chain variants, so it is not a tuning
-  // candidate: it is what runs for G <= kSegs * kSegMax unless a variant is
-  // pinned, and the tuner chooses among variants 0-2 for larger grids only.
-  const bool segable = G <= adi::kSegs * adi::kSegMax;
+  // candidate: it is what runs for G <= 256 (16 segments of 16 elements, the
+  // most that 168 registers hold) unless a variant is pinned, and the tuner
+  // chooses among variants 0-2 for larger grids only.
+  const bool segable = G <= adi::kSegMaxGrid;
   const int forced = f->ctx->tuner.forced[TUNE_ADI];
   if (segable && (forced < 0 || forced == 3)) {
-    auto seg = [&](auto lpw) {
-      constexpr int LPW = decltype(lpw)::value;
-      const int nblk = (G + LPW - 1) / LPW;
-      const int m = (G + adi::kSegs - 1) / adi::kSegs;
-      double* partials = nullptr;
-      if (stats) {
-        const size_t need = static_cast<size_t>(f->nslice) * nblk * 8 + 2 * static_cast<size_t>(f->nslice);
-        if (f->col_partials.size() < need) f->col_partials.alloc(f->ctx, need);
-        partials = f->col_partials.get();
-      }
-      const size_t lds = sizeof(double2) * (5 * static_cast<size_t>(G) + adi::kSegs * LPW);
-      T2* ustar = static_cast<T2*>(adi_ustar(f));
+    const int nblk = (G + adi::kSegLines - 1) / adi::kSegLines;
+    double* partials = nullptr;
+    if (stats) {
+      const size_t need = static_cast<size_t>(f->nslice) * nblk * 8 + 2 * static_cast<size_t>(f->nslice);
+      if (f->col_partials.size() < need) f->col_partials.alloc(f->ctx, need);
+      partials = f->col_partials.get();
+    }
+    T2* ustar = static_cast<T2*>(adi_ustar(f));
+    const double2* tab = f->adi_c + 3 * G;
+    const dim3 block(adi::kSegThreads);
+    const dim3 grid(static_cast<unsigned>((f->nslice + 7) / 8) * 8 * nblk);
+    adi::with_seg_len(G, [&](auto len) {
+      constexpr int K = decltype(len)::value;
       f->ctx->launch(G4H_K_ADI_X, [&] {
-        hipLaunchKernelGGL((adi_x_seg_kernel<P, LPW>), dim3(f->nslice, nblk),
-                           dim3(adi::kSegs * LPW), lds, f->ctx->stream, u, ustar, f->nslice, G,
-                           m, cs, f->adi_c, src, f->src_rect.get(), f->first, add);
+        hipLaunchKernelGGL((adi_x_seg_kernel<P, K>), grid, block, adi::seg_lds_x(K),
+                           f->ctx->stream, u, ustar, f->nslice, nblk, G, cs, tab, src,
+                           f->src_rect.get(), f->first, add);
       });
       f->ctx->launch(G4H_K_ADI_Y, [&] {
-        hipLaunchKernelGGL((adi_y_seg_kernel<P, LPW>), dim3(f->nslice, nblk),
-                           dim3(adi::kSegs * LPW), lds, f->ctx->stream, u, ustar, f->nslice, G,
-                           m, cs, f->adi_c, src, f->src_rect.get(), f->first, add, partials);
+        if (stats)
+          hipLaunchKernelGGL((adi_y_seg_kernel<P, K, true>), grid, block, adi::seg_lds_y(K),
+                             f->ctx->stream, u, ustar, f->nslice, nblk, G, cs, tab, src,
+                             f->src_rect.get(), f->first, add, partials);
+        else
+          hipLaunchKernelGGL((adi_y_seg_kernel<P, K, false>), grid, block, adi::seg_lds_y(K),
+                             f->ctx->stream, u, ustar, f->nslice, nblk, G, cs, tab, src,
+                             f->src_rect.get(), f->first, add, partials);
       });
-      if (stats) field_reduce_partials(f, partials, nblk);
-    };
-    // 64 lines per workgroup (one wave per segment): with 32 (two segments
-    // per wave) the segment bounds are no longer wave-uniform, the element
-    // loops diverge and spill, and the time-dependent G = 151 sweeps ran
-    // 1.5x slower (0.52 against 0.35 ms per x sweep)
-    seg(std::integral_constant<int, 64>{});
+    });
+    if (stats) field_reduce_partials(f, partials, nblk);
     return;
   }
   if (f->adi_y.size() < static_cast<size_t>(f->cells())) f->adi_y.alloc(f->ctx, f->cells());
@@ -631,20 +652,20 @@ void launch_batch_adi_step(Context* ctx, g4h_precision prec, const BatchSegDesc*
                            int nblocks, int k, int gmax, bool add_src, bool stats,
                            bool clear_src) {
   if (nblocks <= 0) return;
-  require(gmax <= adi::kSegs * adi::kSegMax, "segmented sweeps: ngrid above 256");
-  const size_t lds = sizeof(double2) * (5 * static_cast<size_t>(gmax) + adi::kSegs * kLane);
+  require(gmax <= adi::kSegMaxGrid, "segmented sweeps: ngrid above 256");
+  const size_t ldsx = adi::seg_lds_x(adi::seg_len(gmax)), ldsy = adi::seg_lds_y(adi::seg_len(gmax));
   const int src = add_src ? 1 : 0, clr = clear_src ? 1 : 0;
   ctx->launch(G4H_K_ADI_X, [&] {
     if (prec == G4H_FP64)
-      hipLaunchKernelGGL(adi_x_seg_batch_kernel<double>, dim3(nblocks), dim3(adi::kSegs * kLane),
-                         lds, ctx->stream, d_blocks, k, src);
+      hipLaunchKernelGGL(adi_x_seg_batch_kernel<double>, dim3(nblocks), dim3(adi::kSegThreads),
+                         ldsx, ctx->stream, d_blocks, k, src);
     else
-      hipLaunchKernelGGL(adi_x_seg_batch_kernel<float>, dim3(nblocks), dim3(adi::kSegs * kLane),
-                         lds, ctx->stream, d_blocks, k, src);
+      hipLaunchKernelGGL(adi_x_seg_batch_kernel<float>, dim3(nblocks), dim3(adi::kSegThreads),
+                         ldsx, ctx->stream, d_blocks, k, src);
   });
   auto y = [&](auto kern) {
     ctx->launch(G4H_K_ADI_Y, [&] {
-      hipLaunchKernelGGL(kern, dim3(nblocks), dim3(adi::kSegs * kLane), lds, ctx->stream,
+      hipLaunchKernelGGL(kern, dim3(nblocks), dim3(adi::kSegThreads), ldsy, ctx->stream,
                          d_blocks, k, src, clr);
     });
   };
@@ -703,35 +724,46 @@ void adi_prepare(Field* f, double delz) {
       cwet[i] = w1[i - 1] * cbet[i - 1];
       cbet[i] = cd(1.0, 0.0) / (w2[i] - c[i] * cwet[i]);
     }
-    // the segmented sweeps' products over each segment of m elements:
-    // beta_k = prod_(i=s..k) (-c_i cbet_i), delta_k = prod_(i=k+1..e) (-cwet_i),
-    // delta = 0 in the segment that ends the line
-    const int m = (G + adi::kSegs - 1) / adi::kSegs;
-    std::vector<cd> beta(G), delta(G);
-    for (int s0 = 0; s0 < G; s0 += m) {
-      const int e0 = std::min(G, s0 + m);
-      cd b(1.0, 0.0);
-      for (int k = s0; k < e0; ++k) {
-        b = -c[k] * cbet[k] * b;
-        beta[k] = b;
-      }
-      cd d(e0 < G ? -cwet[e0] : cd(0.0, 0.0));
-      for (int k = e0 - 1; k >= s0; --k) {
-        delta[k] = d;
-        if (k > s0) d = -cwet[k] * d;
-      }
-    }
+    // the segmented sweeps' table (adi_seg.hpp)
+    const int K = adi::seg_len(std::min(G, adi::kSegMaxGrid));
+    const bool seg = G <= adi::kSegMaxGrid;
     Field::DelzTable t;
-    t.host.resize(5 * static_cast<size_t>(G));
+    t.host.assign(3 * static_cast<size_t>(G) + (seg ? adi::seg_table_size(K) : 0),
+                  make_double2(0.0, 0.0));
     for (int i = 0; i < G; ++i) {
       t.host[i] = make_double2(c[i].real(), c[i].imag());
       t.host[G + i] = make_double2(cbet[i].real(), cbet[i].imag());
       t.host[2 * G + i] = make_double2(cwet[i].real(), cwet[i].imag());
-      t.host[3 * G + i] = make_double2(beta[i].real(), beta[i].imag());
-      t.host[4 * G + i] = make_double2(delta[i].real(), delta[i].imag());
     }
-    t.dev.alloc(f->ctx, 5 * static_cast<size_t>(G));
-    G4_HIP(hipMemcpyAsync(t.dev.get(), t.host.data(), sizeof(double2) * 5 * G,
+    if (seg) {
+      double2* st = t.host.data() + 3 * G;
+      double mag[adi::kSegs];
+      for (int s = 0; s < adi::kSegs; ++s) {
+        cd prod(1.0, 0.0);
+        for (int j = 0; j < K; ++j) {
+          const int k = s * K + j;
+          const cd cb = k < G ? cbet[k] : cd(0.0, 0.0);
+          st[j * adi::kSegs + s] = make_double2(cb.real(), cb.imag());
+          prod *= cd(0.0, rtmp) * cb;
+        }
+        st[adi::kSegs * K + s] = make_double2(prod.real(), prod.imag());
+        mag[s] = std::abs(prod);
+      }
+      // H: the segments before (after) one whose end values still reach it
+      int H = 1;
+      for (; H < adi::kSegs; ++H) {
+        double worst = 0.0;
+        for (int s = 0; s + H <= adi::kSegs; ++s) {
+          double m = 1.0;
+          for (int i = 0; i < H; ++i) m *= mag[s + i];
+          worst = std::max(worst, m);
+        }
+        if (worst < 1e-25) break;
+      }
+      st[adi::kSegs * K + adi::kSegs] = make_double2(static_cast<double>(H), 0.0);
+    }
+    t.dev.alloc(f->ctx, t.host.size());
+    G4_HIP(hipMemcpyAsync(t.dev.get(), t.host.data(), sizeof(double2) * t.host.size(),
                           hipMemcpyHostToDevice, f->ctx->stream));
     it = f->delz_tables.emplace(key, std::move(t)).first;
   }

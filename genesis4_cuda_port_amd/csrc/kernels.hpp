@@ -69,6 +69,35 @@ __device__ __forceinline__ double2 ld_global(const double2* p) {
 }
 __device__ __forceinline__ double ld_global(const double* p) { return *(gl_d)(p); }
 
+// ---- wave sums ------------------------------------------------------------
+// v of the lane that DPP control CTRL selects (both 32-bit halves moved)
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double((static_cast<long long>(hi) << 32) |
+                              static_cast<unsigned int>(lo));
+}
+__device__ __forceinline__ double lane_f64(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane(static_cast<int>(b), lane);
+  const int hi = __builtin_amdgcn_readlane(static_cast<int>(b >> 32), lane);
+  return __longlong_as_double((static_cast<long long>(hi) << 32) |
+                              static_cast<unsigned int>(lo));
+}
+// Sum of v over the 64 lanes of the wave without LDS: within each row of 16
+// lanes by DPP (lane xor 1, xor 2, then the mirrored lane of the 8 and of the
+// 16, each step pairing lanes whose partial sums cover disjoint halves),
+// then the four row sums read from lanes 0, 16, 32, 48.
+__device__ __forceinline__ double wave_total(double v) {
+  v += dpp_f64<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += dpp_f64<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += dpp_f64<0x141>(v);  // row_half_mirror
+  v += dpp_f64<0x140>(v);  // row_mirror
+  return (lane_f64(v, 0) + lane_f64(v, 16)) + (lane_f64(v, 32) + lane_f64(v, 48));
+}
+
 // ---- particle pass -------------------------------------------------------
 enum Stage : int {
   ST_T1 = 1,     // first transverse half step (with chicane)
@@ -177,7 +206,10 @@ struct BatchRunDesc {
   int K;                       // parts of the run's particle pass (per-step launches)
 };
 
-// One 64-line block of one run's plane for the segmented sweeps of a whole
+// Lines per workgroup of the segmented ADI sweeps.
+constexpr int kAdiSegLines = 16;
+
+// One block of lines of one run's plane for the segmented sweeps of a whole
 // batch in one launch (launch_batch_adi_step).
 struct BatchSegDesc {
   void* u;                     // group field planes (double2* / float2*)
@@ -185,7 +217,7 @@ struct BatchSegDesc {
   const void* src;             // group source planes
   const int4* rect;            // group source rectangles
   double* partials;            // group partials [nrun][nblk][8], then 2 centre values per run
-  const double2* const* adi;   // per step: the group's c, cbet, cwet, beta, delta [5G]
+  const double2* const* adi;   // per step: the group's c, cbet, cwet [3G], then the segment table
   const double* cs;            // per step: the sweeps' i*rtmp coefficient
   int G, nblk, nrun, slice, blk, pad_;
 };
@@ -193,7 +225,7 @@ struct BatchSegDesc {
 // One step k of every run of a batch, each kernel in one launch: the fused
 // particle passes (one workgroup per run, the run's parameter entry of the
 // step), the two segmented sweeps of every run's plane (one workgroup per
-// 64-line block, the run's group tables of the step; G <= 256), and on
+// block of 16 lines, the run's group tables of the step; G <= 256), and on
 // output steps every run's field record from its sweep partials (record r).
 // d_parts: (run, part) of each workgroup, every run's K parts in order.  A
 // split run's parts deposit their out-of-window particles with atomics onto

@@ -63,7 +63,7 @@ g4h_status g4h_context_memory(const g4h_context* ctx, uint64_t* bytes_in_use);
 #define G4H_TUNE_ADI 0   /* 0: workgroup per plane (ngrid <= 360, else as 1),
                             1 / 2: wave per 64 lines, loads 8 / 16 elements
                             ahead; bit-identical results.  3: segmented
-                            sweeps (16 waves per 64 lines, no forward-value
+                            sweeps (16 lanes per line, no forward-value
                             plane; ngrid <= 256, else as 1), results agree
                             with 0-2 to round-off.  Unpinned, 3 runs for
                             ngrid <= 256 and 0-2 are tuned above */

@@ -1,0 +1,61 @@
+"""GPU: segmented ADI sweeps at the edges of their segment lengths.
+
+One field step with the source on against the FP64 oracle at the smallest and
+largest grid of every segment length (4, 7, 8, 10, 13 and 16 elements on 16
+lanes), for slice counts on both sides of the eight XCDs the planes are dealt
+to, and for step lengths from one undulator period to 3000 (coefficient r from
+below 0.1 to above 10, where a line couples over all its segments instead of
+two).  Both sides solve (1 - i r d2) twice; its condition number is
+sqrt(1 + 16 r^2) and a solve rounds within about G eps of it, so the fields
+agree within 4 G eps sqrt(1 + 16 r^2) (MIXED: the field is rounded to FP32
+after each sweep, 4 sqrt(1 + 16 r^2) 2^-24), plus the deposition's own error:
+1e-13 for the order of its FP64 sums, 2e-5 for MIXED's FP32 terms, the bound
+of the other field-step tests."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import _oracle
+from _oracle import OField, dp, ip
+import cases
+from cases import LAMBDA0, quad_step
+from genesis4_cuda_port_amd import api
+
+pytestmark = pytest.mark.gpu
+
+from test_gpu_parity import gpu_beam, gpu_field, noisy_field, relerr  # noqa: E402
+
+
+@pytest.mark.parametrize("prec", [api.FP64, api.MIXED])
+@pytest.mark.parametrize("periods", [1, 300, 3000])
+@pytest.mark.parametrize("ngrid,nslice", [(3, 1), (16, 9), (64, 3), (65, 8), (112, 2), (113, 3),
+                                          (128, 9), (129, 1), (160, 2), (161, 3), (208, 2),
+                                          (209, 1), (256, 3)])
+def test_segment_lengths(ngrid, nslice, periods, prec):
+    print(f"case segments ngrid={ngrid} nslice={nslice} periods={periods} prec={prec}", flush=True)
+    c = cases.make_case(nslice=nslice, npart=256, ngrid=ngrid, seed_power=1e6)
+    st = quad_step()
+    delz = st.delz * periods
+    first = nslice // 2
+    re, im = noisy_field(c, scale=0.1)
+    of = OField(c.nslice, c.ngrid, c.gridmax, LAMBDA0, c.slicelength, 1, re, im, first=first)
+    o = c.beam
+    sre = np.zeros(c.nslice * ngrid * ngrid)
+    sim = np.zeros_like(sre)
+    with api.Context(0) as ctx:
+        f = gpu_field(ctx, c, prec, kind=api.ADI, re=re, im=im, first=first)
+        b = gpu_beam(ctx, c, prec)
+        f.track(b, st, delz)
+        gre, gim, _ = f.download()
+        f.close()
+        b.close()
+    assert _oracle.lib().orc_deposit(c.nslice, ip(o.offsets), dp(o.x), dp(o.y), dp(o.gamma),
+                                     dp(o.theta), of.ptr, st, dp(o.current), delz, dp(sre),
+                                     dp(sim)) == 1
+    _oracle.lib().orc_adi_advance(of.ptr, dp(sre), dp(sim), delz)
+    r = 0.25 * delz / (2 * np.pi / LAMBDA0 * (2 * c.gridmax / (ngrid - 1)) ** 2)
+    eps, dep = (ngrid * 2.0 ** -53, 1e-13) if prec == api.FP64 else (2.0 ** -24, 2e-5)
+    e = relerr(gre + 1j * gim, of.re + 1j * of.im)
+    print(f"  r {r:.3g} rel err {e:.3e}", flush=True)
+    assert e < dep + 4 * eps * np.sqrt(1 + 16 * r * r)
