@@ -325,24 +325,31 @@ bool make_dep(DepParams& d, Field* f, Beam* b, const g4h_step& st, double delz) 
   return true;
 }
 
-// shared by g4h_apply_slippage and the fused run
-int slippage_host(Field* f, double slippage, double sample, int timerun, int periodic) {
-  if (!timerun) return 0;
+// shared by g4h_apply_slippage and the fused run: the ring arithmetic; the
+// caller has the planes brought in zeroed (field_finish)
+Shifted slippage_host(Field* f, double slippage, double sample, int timerun, int periodic) {
+  Shifted z;
+  if (!timerun) return z;
   f->accuslip += slippage;
   const int n = f->nslice;
-  int shifts = 0;
   int direction = 1;
   while (std::abs(f->accuslip) > (sample * 0.8)) {
     direction = f->accuslip < 0 ? -1 : 1;
     f->accuslip -= sample * direction;
     int last = (f->first + n - 1) % n;
     if (direction < 0) last = (last + 1) % n;
-    if (!periodic) field_zero_plane(f, last);
     f->first = last;
     if (direction < 0) f->first = (last + 1) % n;
-    ++shifts;
+    // a shift moves the planes brought in before it along with all others
+    int& in = direction < 0 ? z.back : z.front;
+    int& other = direction < 0 ? z.front : z.back;
+    if (!periodic) {
+      in = std::min(in + 1, n);
+      other = std::max(other - 1, 0);
+    }
+    ++z.shifts;
   }
-  return shifts;
+  return z;
 }
 
 }  // namespace g4
@@ -921,8 +928,9 @@ g4h_status g4h_apply_slippage(g4h_context* ctx, g4h_field* f, double slippage, d
   G4_API_BEGIN
   require(ctx && f, "null argument");
   ctx->activate();
-  const int n = slippage_host(f, slippage, sample, timerun, periodic);
-  if (shifts) *shifts = n;
+  const Shifted z = slippage_host(f, slippage, sample, timerun, periodic);
+  field_finish(f, z, nullptr);
+  if (shifts) *shifts = z.shifts;
   G4_API_END
 }
 
@@ -979,7 +987,7 @@ g4h_status g4h_diag_field_raw(g4h_context* ctx, g4h_field* f, double* raw) {
   const size_t n = static_cast<size_t>(f->nslice) * G4H_FIELD_RAW;
   d.alloc(ctx, n);
   field_plane_stats(f);
-  field_map_stats(f, d.get());
+  field_finish(f, Shifted{}, d.get());
   G4_HIP(hipMemcpyAsync(raw, d.get(), n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   G4_HIP(hipStreamSynchronize(ctx->stream));
   G4_API_END

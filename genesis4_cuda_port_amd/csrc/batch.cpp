@@ -141,7 +141,7 @@ struct g4h_batch {
       p.diag.nharm = nharm;
       launch_particle(g.gctx, g.beam, p);
       field_plane_stats(g.field);
-      field_map_stats(g.field, g.field_hist.get());
+      field_finish(g.field, Shifted{}, g.field_hist.get());
     }
     nrec = 1;
   }
@@ -457,7 +457,8 @@ struct g4h_batch {
       launch_particle(g.gctx, g.beam, g.head[static_cast<size_t>(istep)],
                       g.dtab.get() + static_cast<size_t>(istep) * n);
       field_solve(g.field, g.src_on[static_cast<size_t>(istep)] != 0, out);
-      if (out) field_map_stats(g.field, g.field_hist.get() + static_cast<size_t>(nrec) * field_rec(g));
+      if (out)
+        field_finish(g.field, Shifted{}, g.field_hist.get() + static_cast<size_t>(nrec) * field_rec(g));
     }
     if (out) ++nrec;
   }

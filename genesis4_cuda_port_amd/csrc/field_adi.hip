@@ -507,7 +507,7 @@ __global__ __launch_bounds__(adi::kSegThreads, 3) void adi_y_seg_batch_kernel(
 }
 
 // Field record r of every run from its block partials, summed in block order
-// (as reduce_partials_kernel sums them for a single field).
+// (as field_finish_kernel sums them for a single field).
 __global__ void batch_field_record_kernel(const BatchRunDesc* __restrict__ runs, int nruns,
                                           int r) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -566,11 +566,7 @@ void adi_step(Field* f, bool source_on, bool stats) {
   if (segable && (forced < 0 || forced == 3)) {
     const int nblk = (G + adi::kSegLines - 1) / adi::kSegLines;
     double* partials = nullptr;
-    if (stats) {
-      const size_t need = static_cast<size_t>(f->nslice) * nblk * 8 + 2 * static_cast<size_t>(f->nslice);
-      if (f->col_partials.size() < need) f->col_partials.alloc(f->ctx, need);
-      partials = f->col_partials.get();
-    }
+    if (stats) partials = field_partials(f, nblk);
     T2* ustar = static_cast<T2*>(adi_ustar(f));
     const double2* tab = f->adi_c + 3 * G;
     const dim3 block(adi::kSegThreads);
@@ -593,7 +589,6 @@ void adi_step(Field* f, bool source_on, bool stats) {
                              f->src_rect.get(), f->first, add, partials);
       });
     });
-    if (stats) field_reduce_partials(f, partials, nblk);
     return;
   }
   if (f->adi_y.size() < static_cast<size_t>(f->cells())) f->adi_y.alloc(f->ctx, f->cells());
@@ -603,11 +598,7 @@ void adi_step(Field* f, bool source_on, bool stats) {
   if (variant >= 1) {
     const int nblk = (G + kLane - 1) / kLane;
     double* partials = nullptr;
-    if (stats) {
-      const size_t need = static_cast<size_t>(f->nslice) * nblk * 8 + 2 * static_cast<size_t>(f->nslice);
-      if (f->col_partials.size() < need) f->col_partials.alloc(f->ctx, need);
-      partials = f->col_partials.get();
-    }
+    if (stats) partials = field_partials(f, nblk);
     const size_t ldsc = sizeof(double2) * 3 * static_cast<size_t>(G);
     T2* ustar = static_cast<T2*>(adi_ustar(f));
     auto sweeps = [&](auto ch) {
@@ -628,8 +619,12 @@ void adi_step(Field* f, bool source_on, bool stats) {
       sweeps(std::integral_constant<int, 8>{});
     else
       sweeps(std::integral_constant<int, 16>{});
-    if (stats) field_reduce_partials(f, partials, nblk);
     return;
+  }
+  if (stats) {
+    if (f->plane_stats.size() != static_cast<size_t>(f->nslice) * G4H_FIELD_RAW)
+      f->plane_stats.alloc(f->ctx, static_cast<size_t>(f->nslice) * G4H_FIELD_RAW);
+    f->stats_ntile = 0;
   }
   f->ctx->launch(G4H_K_ADI_X, [&] {
     hipLaunchKernelGGL(adi_x_kernel<P>, dim3(f->nslice), dim3(nt), ldsx, f->ctx->stream, u,

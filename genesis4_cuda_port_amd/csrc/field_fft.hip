@@ -975,11 +975,7 @@ void fft_step(Field* f, bool source_on, bool stats) {
   const double invg = 1.0 / static_cast<double>(G);
   const int ntile = (G + col_tile(G, sizeof(T2)) - 1) / col_tile(G, sizeof(T2));
   double* partials = nullptr;
-  if (stats) {
-    const size_t need = static_cast<size_t>(f->nslice) * ntile * 8 + 2 * static_cast<size_t>(f->nslice);
-    if (f->col_partials.size() < need) f->col_partials.alloc(f->ctx, need);
-    partials = f->col_partials.get();
-  }
+  if (stats) partials = field_partials(f, ntile);
   int add = source_on ? 1 : 0;
   if (source_on && f->filter) {
     // T = 2 IFFT2(filt FFT2(S)) / G^2 into fft_work (ring order)
@@ -997,7 +993,6 @@ void fft_step(Field* f, bool source_on, bool stats) {
   }
   run_rows<P>(f, data, ROW_PROP, invg);
   run_cols<P>(f, data, COL_PROP, invg, add, partials);
-  if (stats) field_reduce_partials(f, partials, ntile);
 }
 
 // The M-point convolution table of a line step with factors P (natural

@@ -10,95 +10,102 @@ void fft_solve(Field* f, bool source_on, bool stats);
 
 namespace {
 
-// Zero ring slot `slot` (ControlCUDA.cpp:237-244 / zero_field_slice_gpu) and
-// flag it so the diagnostics of this step report it as empty.
+// The end of a step: zero fill of the planes that slippage brought in
+// (ControlCUDA.cpp:237-244) and, with raw, the field record of every slice
+// from the solver's per-tile sums, in one launch.  In logical slice order
+// (slice is in ring slot (is + first) % n, DiagnosticCUDA.cpp:320) the new
+// planes are the first `front` and the last `back` slices; their records are
+// zero.  Blocks below nrec take 32 slices each, 8 lanes per slice (lane k
+// adds sum k over the tiles, in tile order; lane 7 copies the centre cell),
+// the others zero planes.  ntile 0: stats holds the slices' sums themselves.
+// Bound: launch latency.  Flag clear, plane fill, tile sums and slice order
+// were four launches of ~4.5 us per step; the tile sums, one thread per
+// slice, took 19 us at 4096 slices x 16 tiles and 33 us at 256 x 64.
 template <class T2>
-__global__ void zero_plane_kernel(T2* u, int64_t plane, int slot, int32_t* zeroed) {
-  T2* p = u + slot * plane;
-  for (int64_t e = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; e < plane;
-       e += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    T2 z;
-    z.x = 0;
-    z.y = 0;
-    p[e] = z;
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) zeroed[slot] = 1;
-}
-
-// raw[is] = plane_stats[(is+first)%n] unless that slot was zeroed since the
-// stats were taken (DiagnosticCUDA.cpp:320 maps storage slot -> logical slice).
-__global__ void map_stats_kernel(const double* ps, const int32_t* zeroed, int n, int first,
-                                 double* raw) {
-  const int is = blockIdx.x * blockDim.x + threadIdx.x;
-  if (is >= n) return;
-  const int p = (is + first) % n;
-  const bool z = zeroed[p] != 0;
-  for (int k = 0; k < G4H_FIELD_RAW; ++k)
-    raw[static_cast<int64_t>(is) * G4H_FIELD_RAW + k] = z ? 0.0 : ps[static_cast<int64_t>(p) * G4H_FIELD_RAW + k];
-}
-
-// partials -> plane_stats[p*9 + k] (k < 7 sums, 7..8 centre)
-__global__ void reduce_partials_kernel(const double* partials, int nslice, int ntile,
-                                       double* plane_stats) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= nslice) return;
-  double* o = plane_stats + static_cast<int64_t>(p) * G4H_FIELD_RAW;
-  for (int k = 0; k < 7; ++k) {
-    double v = 0.0;
-    for (int t = 0; t < ntile; ++t) v += partials[(static_cast<int64_t>(p) * ntile + t) * 8 + k];
+__global__ __launch_bounds__(256) void field_finish_kernel(T2* u, int64_t plane, int n, int first,
+                                                           int front, int back, int nrec,
+                                                           int per_plane, const double* stats,
+                                                           int ntile, double* raw) {
+  if (static_cast<int>(blockIdx.x) < nrec) {
+    const int is = blockIdx.x * 32 + threadIdx.x / 8, k = threadIdx.x % 8;
+    if (is >= n) return;
+    const int p = (is + first) % n;
+    const bool z = is < front || is >= n - back;
+    double* o = raw + static_cast<int64_t>(is) * G4H_FIELD_RAW;
+    double v = 0.0, c = 0.0;
+    if (!z && ntile == 0) {
+      v = stats[static_cast<int64_t>(p) * G4H_FIELD_RAW + k];
+      if (k == 7) c = stats[static_cast<int64_t>(p) * G4H_FIELD_RAW + 8];
+    } else if (!z && k < 7) {
+      const double* t = stats + static_cast<int64_t>(p) * ntile * 8 + k;
+      for (int i = 0; i < ntile; ++i) v += t[i * 8];
+    } else if (!z) {
+      const double* t = stats + static_cast<int64_t>(n) * ntile * 8 + 2 * p;
+      v = t[0];
+      c = t[1];
+    }
     o[k] = v;
+    if (k == 7) o[8] = c;
+    return;
   }
-  o[7] = partials[static_cast<int64_t>(nslice) * ntile * 8 + 2 * p];
-  o[8] = partials[static_cast<int64_t>(nslice) * ntile * 8 + 2 * p + 1];
-}
-
-__global__ void clear_flags_kernel(int32_t* zeroed, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) zeroed[i] = 0;
+  const int b = blockIdx.x - nrec, i = b / per_plane;
+  const int is = i < front ? i : n - back + (i - front);
+  T2* q = u + static_cast<int64_t>((is + first) % n) * plane;
+  T2 z;
+  z.x = 0;
+  z.y = 0;
+  for (int64_t e = (b % per_plane) * 256 + threadIdx.x; e < plane; e += 256 * per_plane) q[e] = z;
 }
 
 // Standalone per-plane field sums (g4_field_slice_reduce_kernel,
-// DiagnosticCUDA.cpp:305-363): one workgroup per ring slot, wave shuffles.
+// DiagnosticCUDA.cpp:305-363) as per-tile sums in the solvers' layout:
+// ntile workgroups per ring slot, whole rows per wave.  Bound: HBM (one
+// read).  One workgroup per plane took 50 us for 48 planes of G = 151 FP64.
 template <class T2>
-__global__ __launch_bounds__(256) void plane_stats_kernel(const T2* u, int G, double* stats) {
+__global__ __launch_bounds__(256) void plane_stats_kernel(const T2* u, int n, int G, int ntile,
+                                                          double* partials) {
   __shared__ double red[4][8];
-  const int p = blockIdx.x;
+  const int p = blockIdx.x / ntile, tile = blockIdx.x % ntile;
   const int64_t plane = static_cast<int64_t>(G) * G;
   const T2* b = u + p * plane;
   const double shift = -0.5 * static_cast<double>(G - 1);
-  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-  for (int64_t e = threadIdx.x; e < plane; e += blockDim.x) {
-    const int iy = static_cast<int>(e / G);
-    const int ix = static_cast<int>(e - static_cast<int64_t>(iy) * G);
-    const double re = b[e].x, im = b[e].y;
-    const double wei = re * re + im * im;
-    const double dx = ix + shift, dy = iy + shift;
-    acc[0] += wei;
-    acc[1] += dx * wei;
-    acc[2] += dx * dx * wei;
-    acc[3] += dy * wei;
-    acc[4] += dy * dy * wei;
-    acc[5] += re;
-    acc[6] += im;
-  }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+  for (int iy = tile * 4 + wave; iy < G; iy += 4 * ntile) {
+    const T2* row = b + static_cast<int64_t>(iy) * G;
+    const double dy = iy + shift;
+    double rw = 0.0;
+    for (int ix = lane; ix < G; ix += 64) {
+      const T2 v = ld_stream(&row[ix]);
+      const double re = v.x, im = v.y;
+      const double wei = re * re + im * im;
+      const double dx = ix + shift;
+      rw += wei;
+      acc[1] += dx * wei;
+      acc[2] += dx * dx * wei;
+      acc[5] += re;
+      acc[6] += im;
+    }
+    acc[0] += rw;
+    acc[3] += dy * rw;
+    acc[4] += dy * dy * rw;
+  }
 #pragma unroll
   for (int k = 0; k < 7; ++k) {
-    double v = acc[k];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    const double v = wave_total(acc[k]);
     if (lane == 0) red[wave][k] = v;
   }
   __syncthreads();
   if (threadIdx.x < 7) {
     double v = 0.0;
     for (int w = 0; w < 4; ++w) v += red[w][threadIdx.x];
-    stats[static_cast<int64_t>(p) * G4H_FIELD_RAW + threadIdx.x] = v;
+    partials[(static_cast<int64_t>(p) * ntile + tile) * 8 + threadIdx.x] = v;
   }
-  if (threadIdx.x == 0) {
-    const int64_t ic = (plane - 1) / 2;
-    stats[static_cast<int64_t>(p) * G4H_FIELD_RAW + 7] = b[ic].x;
-    stats[static_cast<int64_t>(p) * G4H_FIELD_RAW + 8] = b[ic].y;
+  if (tile == 0 && threadIdx.x == 0) {
+    double* c = partials + static_cast<int64_t>(n) * ntile * 8 + 2 * p;
+    const T2 v = b[(plane - 1) / 2];
+    c[0] = v.x;
+    c[1] = v.y;
   }
 }
 
@@ -119,11 +126,11 @@ __global__ void reset_rect_kernel(int4* rect, int4* bbox, int n) {
 
 }  // namespace
 
-void field_reduce_partials(Field* f, const double* partials, int ntile) {
-  f->ctx->launch(G4H_K_OTHER, [&] {
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3((f->nslice + 255) / 256), dim3(256), 0,
-                       f->ctx->stream, partials, f->nslice, ntile, f->plane_stats.get());
-  });
+double* field_partials(Field* f, int ntile) {
+  const size_t need = static_cast<size_t>(f->nslice) * (static_cast<size_t>(ntile) * 8 + 2);
+  if (f->col_partials.size() < need) f->col_partials.alloc(f->ctx, need);
+  f->stats_ntile = ntile;
+  return f->col_partials.get();
 }
 
 void ensure_source(Field* f) {
@@ -163,14 +170,6 @@ void field_reset_source(Field* f) {
     G4_HIP(hipMemsetAsync(f->srcf.get(), 0, sizeof(float2) * f->srcf.size(), f->ctx->stream));
 }
 
-static void ensure_stats(Field* f) {
-  if (f->plane_stats.size() != static_cast<size_t>(f->nslice) * G4H_FIELD_RAW) {
-    f->plane_stats.alloc(f->ctx, static_cast<size_t>(f->nslice) * G4H_FIELD_RAW);
-    f->zeroed.alloc(f->ctx, f->nslice);
-    G4_HIP(hipMemsetAsync(f->zeroed.get(), 0, sizeof(int32_t) * f->nslice, f->ctx->stream));
-  }
-}
-
 void field_prepare_solver(Field* f, double delz) {
   if (f->kind == G4H_SOLVER_FFT)
     fft_prepare(f, delz);
@@ -181,13 +180,6 @@ void field_prepare_solver(Field* f, double delz) {
 
 void field_solve(Field* f, bool source_on, bool stats) {
   ensure_source(f);
-  if (stats) {
-    ensure_stats(f);
-    f->ctx->launch(G4H_K_OTHER, [&] {
-      hipLaunchKernelGGL(clear_flags_kernel, dim3((f->nslice + 255) / 256), dim3(256), 0,
-                         f->ctx->stream, f->zeroed.get(), f->nslice);
-    });
-  }
   if (f->kind == G4H_SOLVER_FFT)
     fft_solve(f, source_on, stats);
   else
@@ -196,33 +188,41 @@ void field_solve(Field* f, bool source_on, bool stats) {
 }
 
 void field_plane_stats(Field* f) {
-  ensure_stats(f);
-  f->ctx->launch(G4H_K_OTHER, [&] {
-    hipLaunchKernelGGL(clear_flags_kernel, dim3((f->nslice + 255) / 256), dim3(256), 0,
-                       f->ctx->stream, f->zeroed.get(), f->nslice);
-  });
+  // enough workgroups to fill the GPU from few planes, at least 4 rows each
+  const int ntile =
+      std::max(1, std::min({16, (1024 + f->nslice - 1) / f->nslice, (f->ngrid + 3) / 4}));
+  double* partials = field_partials(f, ntile);
+  const dim3 grid(static_cast<unsigned>(f->nslice) * ntile);
   f->ctx->launch(G4H_K_OTHER, [&] {
     if (f->prec == G4H_FP64)
-      hipLaunchKernelGGL(plane_stats_kernel<double2>, dim3(f->nslice), dim3(256), 0, f->ctx->stream,
-                         f->ud.get(), f->ngrid, f->plane_stats.get());
+      hipLaunchKernelGGL(plane_stats_kernel<double2>, grid, dim3(256), 0, f->ctx->stream,
+                         f->ud.get(), f->nslice, f->ngrid, ntile, partials);
     else
-      hipLaunchKernelGGL(plane_stats_kernel<float2>, dim3(f->nslice), dim3(256), 0, f->ctx->stream,
-                         f->uf.get(), f->ngrid, f->plane_stats.get());
+      hipLaunchKernelGGL(plane_stats_kernel<float2>, grid, dim3(256), 0, f->ctx->stream,
+                         f->uf.get(), f->nslice, f->ngrid, ntile, partials);
   });
   f->stats_valid = true;
 }
 
-void field_zero_plane(Field* f, int slot) {
-  ensure_stats(f);
+void field_finish(Field* f, const Shifted& z, double* d_raw) {
+  require(!d_raw || f->stats_valid, "field statistics requested before they were computed");
+  const int n = f->nslice;
+  const int front = std::min(z.front, n), back = std::min(z.back, n - front);
+  const int nrec = d_raw ? (n + 31) / 32 : 0;
   const int64_t plane = static_cast<int64_t>(f->ngrid) * f->ngrid;
-  const int blocks = static_cast<int>(std::min<int64_t>(1024, (plane + 255) / 256));
+  const int per_plane = static_cast<int>(std::min<int64_t>(256, (plane + 1023) / 1024));
+  const int64_t blocks = nrec + static_cast<int64_t>(front + back) * per_plane;
+  if (blocks == 0) return;
+  const double* stats = f->stats_ntile == 0 ? f->plane_stats.get() : f->col_partials.get();
   f->ctx->launch(G4H_K_OTHER, [&] {
     if (f->prec == G4H_FP64)
-      hipLaunchKernelGGL(zero_plane_kernel<double2>, dim3(blocks), dim3(256), 0, f->ctx->stream,
-                         f->ud.get(), plane, slot, f->zeroed.get());
+      hipLaunchKernelGGL(field_finish_kernel<double2>, dim3(static_cast<unsigned>(blocks)),
+                         dim3(256), 0, f->ctx->stream, f->ud.get(), plane, n, f->first, front,
+                         back, nrec, per_plane, stats, f->stats_ntile, d_raw);
     else
-      hipLaunchKernelGGL(zero_plane_kernel<float2>, dim3(blocks), dim3(256), 0, f->ctx->stream,
-                         f->uf.get(), plane, slot, f->zeroed.get());
+      hipLaunchKernelGGL(field_finish_kernel<float2>, dim3(static_cast<unsigned>(blocks)),
+                         dim3(256), 0, f->ctx->stream, f->uf.get(), plane, n, f->first, front,
+                         back, nrec, per_plane, stats, f->stats_ntile, d_raw);
   });
 }
 
@@ -238,15 +238,6 @@ void field_copy(Field* dst, const Field* src) {
   dst->first = src->first;
   dst->accuslip = src->accuslip;
   dst->uploaded = true;
-}
-
-void field_map_stats(Field* f, double* d_raw) {
-  require(f->stats_valid, "field statistics requested before they were computed");
-  f->ctx->launch(G4H_K_OTHER, [&] {
-    hipLaunchKernelGGL(map_stats_kernel, dim3((f->nslice + 255) / 256), dim3(256), 0,
-                       f->ctx->stream, f->plane_stats.get(), f->zeroed.get(), f->nslice, f->first,
-                       d_raw);
-  });
 }
 
 }  // namespace g4

@@ -356,9 +356,9 @@ struct Field {
   DevBuf<double> fft_sigmoid;  // [G*G] (filter only)
   DevBuf<double2> fft_work;    // filtered-source work planes (filter only)
   // diagnostics
-  DevBuf<double> plane_stats;  // [nslice * G4H_FIELD_RAW] per ring slot (last solve)
-  DevBuf<double> col_partials; // FFT column-tile partial sums
-  DevBuf<int32_t> zeroed;      // [nslice] ring slots zeroed by slippage since last map
+  DevBuf<double> plane_stats;   // [nslice * G4H_FIELD_RAW] per ring slot (stats_ntile 0)
+  DevBuf<double> col_partials;  // per-tile field sums
+  int stats_ntile = 0;          // tiles per plane of the last sums
   bool stats_valid = false;
 
   int64_t cells() const { return static_cast<int64_t>(nslice) * ngrid * ngrid; }

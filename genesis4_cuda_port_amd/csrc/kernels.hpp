@@ -289,15 +289,23 @@ bool make_dep(DepParams& d, Field* f, Beam* b, const g4h_step& st, double delz);
 void field_prepare_solver(Field* f, double delz);  // (re)build coefficient tables
 void* field_adi_ustar(Field* f);  // the ADI x sweep's output planes (allocated on first use)
 // One field step with the source (if source_on).  When stats != 0 the last
-// pass also writes per-ring-slot field sums into f->plane_stats.
+// pass also writes the planes' field sums: per-tile sums in f->col_partials
+// (stats_ntile tiles; field_partials), or whole ones in f->plane_stats
+// (stats_ntile 0).
 void field_solve(Field* f, bool source_on, bool stats);
 void field_plane_stats(Field* f);                      // standalone field sums
-// Per-tile partial field sums partials[(p*ntile + t)*8 + k] (k < 7) and the
-// centre cell at partials[nslice*ntile*8 + 2p] -> plane_stats, tiles in order.
-void field_reduce_partials(Field* f, const double* partials, int ntile);
-void field_zero_plane(Field* f, int slot);             // slippage zero fill
-// plane_stats (ring order) -> raw[nslice*9] (logical order), honouring zeroed slots.
-void field_map_stats(Field* f, double* d_raw);
+// Room for per-tile field sums partials[(p*ntile + t)*8 + k] (k < 7) and the
+// centre cells at partials[nslice*ntile*8 + 2p]; makes them the planes' sums.
+double* field_partials(Field* f, int ntile);
+// Slippage (ring arithmetic on the host only): the slices whose planes it
+// brought in empty, counted from either end of the logical order.
+struct Shifted {
+  int front = 0, back = 0, shifts = 0;
+};
+Shifted slippage_host(Field* f, double slippage, double sample, int timerun, int periodic);
+// Zero fill of the planes that slippage brought in and, with d_raw, the
+// record of the solve's field sums: raw[nslice*9] in logical order.
+void field_finish(Field* f, const Shifted& z, double* d_raw);
 // source bookkeeping reset (new beam or new source allocation)
 void field_reset_source(Field* f);
 void field_copy(Field* dst, const Field* src);

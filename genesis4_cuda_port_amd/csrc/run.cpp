@@ -9,9 +9,9 @@
 //      FieldSolver*::advance + DiagnosticCUDA beam kernel);
 //   2. the field solver passes (FFT rows+columns or ADI x+y sweeps), the last
 //      one reducing the per-plane field sums on output steps;
-//   3. the slippage ring shift (host integer update + zero fill of the
-//      incoming plane);
-//   4. on output steps, the map of per-plane field sums to logical slices.
+//   3. the slippage ring shift (host integer update), then one launch that
+//      zeroes the incoming plane and, on output steps, writes the slices'
+//      field records from the solver's per-tile sums.
 // Diagnostics stay in device history buffers until g4h_run_download_diag.
 //
 // Ensembles (the same lattice and shapes run again with a new beam or seed:
@@ -26,7 +26,6 @@
 #include "kernels.hpp"
 
 namespace g4 {
-int slippage_host(Field* f, double slippage, double sample, int timerun, int periodic);
 void context_child_added(Context* c);
 void context_child_removed(Context* c);
 }
@@ -75,7 +74,7 @@ struct g4h_run {
     p.diag.nharm = cfg.nharm;
     launch_particle(ctx, b, p);
     field_plane_stats(f);
-    field_map_stats(f, field_hist.get() + nrec * field_rec());
+    field_finish(f, Shifted{}, field_hist.get() + nrec * field_rec());
     ++nrec;
   }
 
@@ -118,9 +117,9 @@ struct g4h_run {
     }
     launch_particle(ctx, b, p);
     field_solve(f, src_on, out);
-    slippage_host(f, st.slippage, cfg.sample, cfg.timerun, cfg.periodic);
+    const Shifted z = slippage_host(f, st.slippage, cfg.sample, cfg.timerun, cfg.periodic);
+    field_finish(f, z, out ? field_hist.get() + nrec * field_rec() : nullptr);
     if (out) {
-      field_map_stats(f, field_hist.get() + nrec * field_rec());
       if (b->ef.nz > 0 && sc_hist.size() >= static_cast<size_t>(nrec + 1) * b->nslice)
         G4_HIP(hipMemcpyAsync(sc_hist.get() + static_cast<size_t>(nrec) * b->nslice,
                               b->scrms.get(), sizeof(double) * b->nslice,
