@@ -1,5 +1,6 @@
 // abi.cpp - the g4hip C ABI: state objects, step operators, diagnostics.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -15,6 +16,11 @@ thread_local std::string g_last_error;
 }
 void context_child_added(Context* c);
 void context_child_removed(Context* c);
+
+void Beam::touched() {
+  static std::atomic<uint64_t> last{0};
+  epoch = ++last;
+}
 
 void set_last_error(const std::string& m) { g_last_error = m; }
 
@@ -506,6 +512,7 @@ g4h_status g4h_beam_set_current(g4h_beam* b, const double* current) {
   require(b && current, "null argument");
   b->ctx->activate();
   b->current_h.assign(current, current + b->nslice);
+  b->touched();
   std::vector<double> con(b->nslice);
   for (int s = 0; s < b->nslice; ++s) {
     const int np = b->off_h[s + 1] - b->off_h[s];
@@ -545,6 +552,7 @@ g4h_status g4h_beam_upload(g4h_beam* b, const double* x, const double* y, const 
     G4_HIP(hipMemcpy(b->theta.get(), theta, n * 8, hipMemcpyHostToDevice));
   }
   b->uploaded = true;
+  b->touched();
   G4_API_END
 }
 
@@ -918,8 +926,13 @@ g4h_status g4h_field_track(g4h_context* ctx, g4h_field* f, g4h_beam* b, const g4
   p.gamma0 = b->gamma_ref;
   p.stages = ST_DEP;
   const bool on = make_dep(p.dep, f, b, *und, delz) && b->np > 0;
-  if (on) launch_particle(ctx, b, p);
-  field_solve(f, on, false);
+  if (on) {
+    ParticleLaunch how;
+    how.prepass = source_needs_prepass(f, b);
+    launch_particle(ctx, b, p, how);
+    source_deposited(f, b);
+  }
+  field_solve(f, on, false, split_of(ctx, b) > 1);
   G4_API_END
 }
 

@@ -454,8 +454,9 @@ struct g4h_batch {
     for (Group& g : groups) {
       const size_t n = g.runs.size();
       field_prepare_solver(g.field, st0.delz);
-      launch_particle(g.gctx, g.beam, g.head[static_cast<size_t>(istep)],
-                      g.dtab.get() + static_cast<size_t>(istep) * n);
+      ParticleLaunch how;
+      how.d_table = g.dtab.get() + static_cast<size_t>(istep) * n;
+      launch_particle(g.gctx, g.beam, g.head[static_cast<size_t>(istep)], how);
       field_solve(g.field, g.src_on[static_cast<size_t>(istep)] != 0, out);
       if (out)
         field_finish(g.field, Shifted{}, g.field_hist.get() + static_cast<size_t>(nrec) * field_rec(g));

@@ -419,7 +419,7 @@ template <class P, int K, bool STATS>
 __global__ __launch_bounds__(adi::kSegThreads, K > 10 ? 3 : 4) void adi_y_seg_kernel(
     typename A2<P>::T* u, const typename A2<P>::T* ustar, int nslice, int nblk, int G, double cs,
     const double2* __restrict__ tab, const typename A2<P>::T* src, const int4* rect, int first,
-    int add_src, double* partials) {
+    int add_src, int clear_src, double* partials) {
   using T2 = typename A2<P>::T;
   extern __shared__ double2 lds[];
   const SegBlock b = seg_block(nblk);
@@ -439,7 +439,8 @@ __global__ __launch_bounds__(adi::kSegThreads, K > 10 ? 3 : 4) void adi_y_seg_ke
   double* part = STATS ? partials + (static_cast<int64_t>(b.p) * nblk + b.blk) * 8 : nullptr;
   double* centre = STATS ? partials + static_cast<int64_t>(nslice) * nblk * 8 + 2 * b.p : nullptr;
   adi::seg_y<P, K, STATS>(ustar + b.p * plane, u + b.p * plane, G, cs, lds, sp, rc, b.blk, ends,
-                          red, part, centre, nullptr);
+                          red, part, centre,
+                          clear_src ? const_cast<T2*>(sp) : nullptr);
 }
 
 // The segmented sweeps of every run of a batch in one launch: workgroup b
@@ -538,7 +539,7 @@ void* adi_ustar(Field* f) {
 }
 
 template <class P>
-void adi_step(Field* f, bool source_on, bool stats) {
+void adi_step(Field* f, bool source_on, bool stats, bool clear) {
   using T2 = typename A2<P>::T;
   const int G = f->ngrid;
   const int nt = ((G + 63) / 64) * 64;
@@ -570,6 +571,7 @@ void adi_step(Field* f, bool source_on, bool stats) {
     T2* ustar = static_cast<T2*>(adi_ustar(f));
     const double2* tab = f->adi_c + 3 * G;
     const dim3 block(adi::kSegThreads);
+    const int clr = clear ? 1 : 0;
     const dim3 grid(static_cast<unsigned>((f->nslice + 7) / 8) * 8 * nblk);
     adi::with_seg_len(G, [&](auto len) {
       constexpr int K = decltype(len)::value;
@@ -582,13 +584,14 @@ void adi_step(Field* f, bool source_on, bool stats) {
         if (stats)
           hipLaunchKernelGGL((adi_y_seg_kernel<P, K, true>), grid, block, adi::seg_lds_y(K),
                              f->ctx->stream, u, ustar, f->nslice, nblk, G, cs, tab, src,
-                             f->src_rect.get(), f->first, add, partials);
+                             f->src_rect.get(), f->first, add, clr, partials);
         else
           hipLaunchKernelGGL((adi_y_seg_kernel<P, K, false>), grid, block, adi::seg_lds_y(K),
                              f->ctx->stream, u, ustar, f->nslice, nblk, G, cs, tab, src,
-                             f->src_rect.get(), f->first, add, partials);
+                             f->src_rect.get(), f->first, add, clr, partials);
       });
     });
+    if (clear) f->src_clear = true;
     return;
   }
   if (f->adi_y.size() < static_cast<size_t>(f->cells())) f->adi_y.alloc(f->ctx, f->cells());
@@ -769,11 +772,11 @@ void adi_prepare(Field* f, double delz) {
   f->adi_delz = delz;
 }
 
-void adi_solve(Field* f, bool source_on, bool stats) {
+void adi_solve(Field* f, bool source_on, bool stats, bool clear) {
   if (f->prec == G4H_FP64)
-    adi_step<double>(f, source_on, stats);
+    adi_step<double>(f, source_on, stats, clear);
   else
-    adi_step<float>(f, source_on, stats);
+    adi_step<float>(f, source_on, stats, clear);
 }
 
 }  // namespace g4

@@ -406,8 +406,8 @@ template <class P, int G>
 __global__ __launch_bounds__((RegCfg<P, G>::kThreads),
                              (RegCfg<P, G>::kMinWaves)) void fft_cols_reg_kernel(
     typename C2<P>::T* u, int nslice, const double2* tw_d, const double2* mult_d,
-    const double* sigmoid, int mode, double scale, const typename C2<P>::T* src, const int4* rect,
-    int first, int add_src, const double2* work, double* partials) {
+    const double* sigmoid, int mode, double scale, typename C2<P>::T* src, const int4* rect,
+    int first, int add_src, int clear_src, const double2* work, double* partials) {
   using T2 = typename C2<P>::T;
   using S = fftr::Shape<G>;
   using C = RegCfg<P, G>;
@@ -474,29 +474,15 @@ __global__ __launch_bounds__((RegCfg<P, G>::kThreads),
   const int s = ((p - first) % nslice + nslice) % nslice;  // beam slice of this ring plane
   int4 rc = make_int4(0, 0, 0, 0);
   if (add_src == 1) rc = rect[s];
-  const T2* sp = (add_src == 1) ? src + static_cast<int64_t>(s) * G * G : nullptr;
+  T2* sp = (add_src == 1) ? src + static_cast<int64_t>(s) * G * G : nullptr;
   const double2* wp = (add_src == 2) ? work + static_cast<int64_t>(p) * G * G : nullptr;
   const double shift = -0.5 * static_cast<double>(G - 1);
-  const int64_t icenter = (static_cast<int64_t>(G) * G - 1) / 2;
+  const T2 zero = T2{};
+  constexpr int crow = (G * G - 1) / 2 / G, ccol = (G * G - 1) / 2 % G;  // centre cell
   const bool src_col = sp && c >= rc.x && c < rc.z;
   double acc[7] = {0, 0, 0, 0, 0, 0, 0};
   if constexpr (kDirect) {
     const double dx = c + shift;
-    // the stored value of cell (row, this thread's column)
-    auto out = [&](int row, int64_t gi, T2 o) {
-      o.x *= sc;
-      o.y *= sc;
-      if (src_col && row >= rc.y && row < rc.w) {
-        const T2 sv = ld_stream(&sp[gi]);
-        o.x += P(2) * sv.x;
-        o.y += P(2) * sv.y;
-      } else if (wp) {
-        const double2 wv = ld_stream(&wp[gi]);
-        o.x += static_cast<P>(wv.x);
-        o.y += static_cast<P>(wv.y);
-      }
-      return o;
-    };
     // The thread's column is fixed, so its x moments are dx and dx^2 times
     // its sum of |u|^2, taken once after the loop.  MIXED sums its R
     // cells in FP32 (as the particle pass sums its moments per thread); the
@@ -507,8 +493,26 @@ __global__ __launch_bounds__((RegCfg<P, G>::kThreads),
       constexpr int r = decltype(ic)::value;
       const int row = t + L * r;
       const int64_t gi = static_cast<int64_t>(row) * G + c;
-      const T2 o = out(row, gi, v[r]);
+      T2 o = v[r];
+      o.x *= sc;
+      o.y *= sc;
+      if (src_col && row >= rc.y && row < rc.w) {
+        const T2 sv = ld_stream(&sp[gi]);
+        o.x += P(2) * sv.x;
+        o.y += P(2) * sv.y;
+        if (clear_src) sp[gi] = zero;
+      } else if (wp) {
+        const double2 wv = ld_stream(&wp[gi]);
+        o.x += static_cast<P>(wv.x);
+        o.y += static_cast<P>(wv.y);
+      }
       st_stream(&plane[gi], o);
+      if constexpr (r == crow / L) {
+        if (partials && c == ccol && t == crow % L) {
+          partials[static_cast<int64_t>(nslice) * ntile * 8 + 2 * p] = o.x;
+          partials[static_cast<int64_t>(nslice) * ntile * 8 + 2 * p + 1] = o.y;
+        }
+      }
       if (partials) {
         const A re = o.x, im = o.y;
         const A wei = re * re + im * im;
@@ -528,13 +532,6 @@ __global__ __launch_bounds__((RegCfg<P, G>::kThreads),
       acc[4] = s4;
       acc[5] = s5;
       acc[6] = s6;
-      // the centre cell, recomputed as stored by the thread that holds it
-      constexpr int crow = (G * G - 1) / 2 / G, ccol = (G * G - 1) / 2 % G;
-      if (c == ccol && t == crow % L) {
-        const T2 o = out(crow, icenter, v[crow / L]);
-        partials[static_cast<int64_t>(nslice) * ntile * 8 + 2 * p] = o.x;
-        partials[static_cast<int64_t>(nslice) * ntile * 8 + 2 * p + 1] = o.y;
-      }
     }
   } else if (valid) {
     const double dx = c + shift;
@@ -549,6 +546,7 @@ __global__ __launch_bounds__((RegCfg<P, G>::kThreads),
         const T2 sv = sp[gi];
         o.x += P(2) * sv.x;
         o.y += P(2) * sv.y;
+        if (clear_src) sp[gi] = zero;
       } else if (wp) {
         const double2 wv = wp[gi];
         o.x += static_cast<P>(wv.x);
@@ -566,7 +564,7 @@ __global__ __launch_bounds__((RegCfg<P, G>::kThreads),
         acc[4] += dy * dy * wei;
         acc[5] += re;
         acc[6] += im;
-        if (gi == icenter) {
+        if (row == crow && c == ccol) {
           partials[static_cast<int64_t>(nslice) * ntile * 8 + 2 * p] = re;
           partials[static_cast<int64_t>(nslice) * ntile * 8 + 2 * p + 1] = im;
         }
@@ -697,8 +695,8 @@ __global__ __launch_bounds__((ConvCfg<P, M>::kThreads)) void fft_rows_conv_kerne
 template <class P, int M>
 __global__ __launch_bounds__((ConvCfg<P, M>::kThreads)) void fft_cols_conv_kernel(
     typename C2<P>::T* u, int nslice, int N, const double2* tw_d, const double2* mult_d,
-    const typename C2<P>::T* src, const int4* rect, int first, int add_src, const double2* work,
-    double* partials) {
+    typename C2<P>::T* src, const int4* rect, int first, int add_src, int clear_src,
+    const double2* work, double* partials) {
   using T2 = typename C2<P>::T;
   using S = fftr::Shape<M>;
   using C = ConvCfg<P, M>;
@@ -739,7 +737,7 @@ __global__ __launch_bounds__((ConvCfg<P, M>::kThreads)) void fft_cols_conv_kerne
   const int s = ((p - first) % nslice + nslice) % nslice;  // beam slice of this ring plane
   int4 rc = make_int4(0, 0, 0, 0);
   if (add_src == 1) rc = rect[s];
-  const T2* sp = (add_src == 1) ? src + static_cast<int64_t>(s) * N * N : nullptr;
+  T2* sp = (add_src == 1) ? src + static_cast<int64_t>(s) * N * N : nullptr;
   const double2* wp = (add_src == 2) ? work + static_cast<int64_t>(p) * N * N : nullptr;
   const bool scol = sp && col >= rc.x && col < rc.z;
   const double shift = -0.5 * static_cast<double>(N - 1);
@@ -758,6 +756,7 @@ __global__ __launch_bounds__((ConvCfg<P, M>::kThreads)) void fft_cols_conv_kerne
           const T2 sv = ld_stream(&sp[gi]);
           o.x += P(2) * sv.x;
           o.y += P(2) * sv.y;
+          if (clear_src) sp[gi] = T2{};
         } else if (wp) {
           const double2 wv = ld_stream(&wp[gi]);
           o.x += static_cast<P>(wv.x);
@@ -842,15 +841,15 @@ void rows_reg(Field* f, typename C2<P>::T* data, int mode, double scale) {
 }
 
 template <class P, int G>
-void cols_reg(Field* f, typename C2<P>::T* data, int mode, double scale, int add_src,
+void cols_reg(Field* f, typename C2<P>::T* data, int mode, double scale, int add_src, int clear,
               double* partials) {
   using T2 = typename C2<P>::T;
   using C = RegCfg<P, G>;
   constexpr int ntile = G / C::kTile;
   hipLaunchKernelGGL((fft_cols_reg_kernel<P, G>), dim3(f->nslice * ntile), dim3(C::kThreads), 0,
                      f->ctx->stream, data, f->nslice, f->fft_tw.get(), f->fft_prop,
-                     f->fft_sigmoid.get(), mode, scale, static_cast<const T2*>(f->src()),
-                     f->src_rect.get(), f->first, add_src, f->fft_work.get(), partials);
+                     f->fft_sigmoid.get(), mode, scale, static_cast<T2*>(f->src()),
+                     f->src_rect.get(), f->first, add_src, clear, f->fft_work.get(), partials);
 }
 
 template <class P, int M>
@@ -867,14 +866,14 @@ void rows_conv(Field* f, typename C2<P>::T* data) {
 }
 
 template <class P, int M>
-void cols_conv(Field* f, typename C2<P>::T* data, int add_src, double* partials) {
+void cols_conv(Field* f, typename C2<P>::T* data, int add_src, int clear, double* partials) {
   using T2 = typename C2<P>::T;
   using C = ConvCfg<P, M>;
   const int N = f->ngrid;
   const int ntile = (N + ConvCfg<P, M>::TW - 1) / ConvCfg<P, M>::TW;
   hipLaunchKernelGGL((fft_cols_conv_kernel<P, M>), dim3(f->nslice * ntile), dim3(C::kThreads), 0,
                      f->ctx->stream, data, f->nslice, N, f->fft_tw_conv.get(), f->fft_prop,
-                     static_cast<const T2*>(f->src()), f->src_rect.get(), f->first, add_src,
+                     static_cast<T2*>(f->src()), f->src_rect.get(), f->first, add_src, clear,
                      f->fft_work.get(), partials);
 }
 
@@ -940,19 +939,22 @@ void run_rows(Field* f, typename C2<P>::T* data, int mode, double scale) {
 
 template <class P>
 void run_cols(Field* f, typename C2<P>::T* data, int mode, double scale, int add_src,
-              double* partials) {
+              double* partials, bool clear = false) {
   using T2 = typename C2<P>::T;
   const int G = f->ngrid;
+  // the register passes can zero the source cells that they add
+  clear = clear && add_src == 1 && mode == COL_PROP && (is_pow2(G) || conv_points(G));
+  const int clr = clear ? 1 : 0;
   f->ctx->launch(G4H_K_FFT_COLS, [&] {
     if (is_pow2(G)) {
       with_pow2(G, [&](auto g) {
-        cols_reg<P, decltype(g)::value>(f, data, mode, scale, add_src, partials);
+        cols_reg<P, decltype(g)::value>(f, data, mode, scale, add_src, clr, partials);
       });
       return;
     }
     if (mode == COL_PROP && conv_points(G)) {
       with_pow2(conv_points(G), [&](auto m) {
-        cols_conv<P, decltype(m)::value>(f, data, add_src, partials);
+        cols_conv<P, decltype(m)::value>(f, data, add_src, clr, partials);
       });
       return;
     }
@@ -965,10 +967,11 @@ void run_cols(Field* f, typename C2<P>::T* data, int mode, double scale, int add
                        static_cast<const T2*>(f->src()), f->src_rect.get(), f->first, add_src,
                        f->fft_work.get(), partials);
   });
+  if (clear) f->src_clear = true;
 }
 
 template <class P>
-void fft_step(Field* f, bool source_on, bool stats) {
+void fft_step(Field* f, bool source_on, bool stats, bool clear) {
   using T2 = typename C2<P>::T;
   const int G = f->ngrid;
   T2* data = static_cast<T2*>(f->data());
@@ -992,7 +995,7 @@ void fft_step(Field* f, bool source_on, bool stats) {
     add = 2;
   }
   run_rows<P>(f, data, ROW_PROP, invg);
-  run_cols<P>(f, data, COL_PROP, invg, add, partials);
+  run_cols<P>(f, data, COL_PROP, invg, add, partials, clear);
 }
 
 // The M-point convolution table of a line step with factors P (natural
@@ -1126,11 +1129,11 @@ void fft_prepare(Field* f, double delz) {
   }
 }
 
-void fft_solve(Field* f, bool source_on, bool stats) {
+void fft_solve(Field* f, bool source_on, bool stats, bool clear) {
   if (f->prec == G4H_FP64)
-    fft_step<double>(f, source_on, stats);
+    fft_step<double>(f, source_on, stats, clear);
   else
-    fft_step<float>(f, source_on, stats);
+    fft_step<float>(f, source_on, stats, clear);
 }
 
 bool fft_supported(int G) { return G >= 2 && G <= 1024; }

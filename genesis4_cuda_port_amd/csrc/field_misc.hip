@@ -4,9 +4,9 @@
 namespace g4 {
 
 void adi_prepare(Field* f, double delz);
-void adi_solve(Field* f, bool source_on, bool stats);
+void adi_solve(Field* f, bool source_on, bool stats, bool clear);
 void fft_prepare(Field* f, double delz);
-void fft_solve(Field* f, bool source_on, bool stats);
+void fft_solve(Field* f, bool source_on, bool stats, bool clear);
 
 namespace {
 
@@ -157,7 +157,18 @@ void ensure_source(Field* f) {
   if (fresh) field_reset_source(f);
 }
 
+bool source_needs_prepass(const Field* f, const Beam* b) {
+  return !f->src_clear || f->src_epoch != b->epoch;
+}
+
+void source_deposited(Field* f, const Beam* b) {
+  f->src_clear = false;
+  f->src_epoch = b->epoch;
+}
+
 void field_reset_source(Field* f) {
+  f->src_clear = false;
+  f->src_epoch = 0;
   if (f->src_rect.empty()) return;
   f->ctx->launch(G4H_K_OTHER, [&] {
     hipLaunchKernelGGL(reset_rect_kernel, dim3((f->nslice + 255) / 256), dim3(256), 0,
@@ -178,12 +189,12 @@ void field_prepare_solver(Field* f, double delz) {
   f->solver_ready = true;
 }
 
-void field_solve(Field* f, bool source_on, bool stats) {
+void field_solve(Field* f, bool source_on, bool stats, bool clear) {
   ensure_source(f);
   if (f->kind == G4H_SOLVER_FFT)
-    fft_solve(f, source_on, stats);
+    fft_solve(f, source_on, stats, clear && source_on);
   else
-    adi_solve(f, source_on, stats);
+    adi_solve(f, source_on, stats, clear && source_on);
   f->stats_valid = stats;
 }
 

@@ -269,6 +269,10 @@ struct Beam {
   int64_t np = 0;
   double gamma_ref = 0.0;
   bool uploaded = false;
+  // Changes (to a value no beam had before) when positions or currents are
+  // set from outside: slices may then need new deposition footprints.
+  uint64_t epoch = 0;
+  void touched();
   std::vector<int32_t> off_h;
   std::vector<double> current_h;
   DevBuf<int32_t> off;           // [nslice+1]
@@ -311,6 +315,8 @@ struct Field {
   DevBuf<float2> srcf;
   DevBuf<int4> src_rect;  // [nslice] half-open (x0,y0,x1,y1) of possibly nonzero cells
   DevBuf<int4> dep_bbox;  // [nslice] (minx,miny,maxx,maxy) of the cells deposited last step
+  bool src_clear = false;   // the last solve zeroed the source behind itself
+  uint64_t src_epoch = 0;   // Beam::epoch of the last deposition (0: none since a reset)
   // solver
   g4h_solver_kind kind = G4H_SOLVER_ADI;
   bool filter = false;

@@ -171,11 +171,24 @@ struct ParticleParams {
   DiagParams diag;
 };
 
-// With d_table (device, one entry per slice) each slice's workgroup takes its
-// parameters from the table; p still selects the kernel variant (stages,
-// field count, harmonics, window size), which must be common to all entries.
+// How a particle pass is launched.  With d_table (device, one entry per
+// slice) each slice's workgroup takes its parameters from the table; p still
+// selects the kernel variant (stages, field count, harmonics, window size),
+// which must be common to all entries.  d_prm: p's own copy in device memory,
+// where the caller has one (FP64).  prepass: a deposition split over several
+// workgroups per slice first zeroes the old source rectangles and takes
+// missing footprints from the current positions; not needed when the source
+// is known to be clear and its footprints to be of this beam
+// (source_needs_prepass).
+struct ParticleLaunch {
+  const ParticleParams* d_table = nullptr;
+  const ParticleParams* d_prm = nullptr;
+  bool prepass = true;
+};
 void launch_particle(Context* ctx, Beam* b, const ParticleParams& p,
-                     const ParticleParams* d_table = nullptr);
+                     const ParticleLaunch& how = {});
+// Workgroups per slice of a particle pass over the beam.
+int split_of(Context* ctx, const Beam* b);
 void launch_cell_index(Context* ctx, Beam* b, const Field* f, int32_t* d_cell);
 // One run of a persistent batch launch (launch_batch_persistent): where its
 // slice lives in its group's beam and field, and its group's per-step tables.
@@ -291,8 +304,9 @@ void* field_adi_ustar(Field* f);  // the ADI x sweep's output planes (allocated 
 // One field step with the source (if source_on).  When stats != 0 the last
 // pass also writes the planes' field sums: per-tile sums in f->col_partials
 // (stats_ntile tiles; field_partials), or whole ones in f->plane_stats
-// (stats_ntile 0).
-void field_solve(Field* f, bool source_on, bool stats);
+// (stats_ntile 0).  clear: zero the source cells behind the last pass that
+// reads them, where that pass can (f->src_clear tells).
+void field_solve(Field* f, bool source_on, bool stats, bool clear = false);
 void field_plane_stats(Field* f);                      // standalone field sums
 // Room for per-tile field sums partials[(p*ntile + t)*8 + k] (k < 7) and the
 // centre cells at partials[nslice*ntile*8 + 2p]; makes them the planes' sums.
@@ -306,6 +320,10 @@ Shifted slippage_host(Field* f, double slippage, double sample, int timerun, int
 // Zero fill of the planes that slippage brought in and, with d_raw, the
 // record of the solve's field sums: raw[nslice*9] in logical order.
 void field_finish(Field* f, const Shifted& z, double* d_raw);
+// Whether a split deposition of the beam onto the field needs its pre-pass,
+// and the bookkeeping of a deposition launched after asking.
+bool source_needs_prepass(const Field* f, const Beam* b);
+void source_deposited(Field* f, const Beam* b);
 // source bookkeeping reset (new beam or new source allocation)
 void field_reset_source(Field* f);
 void field_copy(Field* dst, const Field* src);

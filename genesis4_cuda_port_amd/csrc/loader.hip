@@ -87,6 +87,7 @@ g4h_status g4h_beam_generate(g4h_beam* b, const g4h_beam_spec* spec, const doubl
                          b->pyf.get(), b->gf.get(), b->theta.get());
   });
   b->uploaded = true;
+  b->touched();
   // the slice currents buffer is released after the kernel (stream-ordered)
   G4_API_END
 }

@@ -22,11 +22,12 @@
 //
 // Few slices (steady-state batches, short time windows) would leave most
 // CUs idle, so such a pass is split: K workgroups per slice (gridDim.y) each
-// take a contiguous part of its particles with the same window placement,
-// write their window and sums to scratch, and the last to arrive (an atomic
-// counter per slice) adds the K windows in part order and writes the plane
-// and the slice's sums.  The previous source rectangle is then zeroed by a
-// pass before, so the fallback atomics of every part land on cleared cells.
+// take a contiguous part of its particles with the same window placement and
+// write their window, boxes and sums to scratch; a second launch adds the K
+// windows in part order and writes the plane, the slice's boxes and sums.
+// The fallback atomics of every part need a cleared source plane: the solver
+// pass that reads the source last clears it behind itself (field_solve's
+// clear), and a pre-pass does where that has not happened (launch_particle).
 //
 // MIXED arithmetic: x, y, px, py and dgamma = gamma - gamma_ref in FP32,
 // theta in FP64.  The phase equation theta' = xks(1 - 1/beta_par) + xku is
@@ -868,6 +869,8 @@ struct SplitScratch {
   double2* win;  // [nslice][K][window_cap]
   double* red;   // [nslice][K][kRedStride]
   int4* fb;      // [nslice][K]
+  int4* tb;      // [nslice][K] box of each part's non-zero window cells
+  int4* wb;      // [nslice] the parts' common window (x0, y0, width, height)
   int own;       // nonzero: the arrays are this slice's own ([K][..])
   // nonzero: each part adds its window to the (cleared) source plane with
   // atomics and folds its boxes into fb[0] (non-zero cells) and fb[1] (the
@@ -1357,8 +1360,28 @@ __device__ __forceinline__ void particle_slice(BeamPtr<P> b, const int32_t* off,
         }
       } else {
         double2* w = sp.win + part * prm.dep.window_cap;
-        for (int k = tid; k < ww * wh; k += NT) w[k] = win[k];
-        if (tid == 0) sp.fb[part] = make_int4(s_fb[0], s_fb[1], s_fb[2], s_fb[3]);
+        int mnx = 0x7fffffff, mny = 0x7fffffff, mxx = -1, mxy = -1;
+        for (int k = tid; k < ww * wh; k += NT) {
+          const double2 v = win[k];
+          w[k] = v;
+          if (v.x != 0.0 || v.y != 0.0) {
+            const int cy = wy0 + k / ww, cx = wx0 + k % ww;
+            mnx = min(mnx, cx);
+            mny = min(mny, cy);
+            mxx = max(mxx, cx);
+            mxy = max(mxy, cy);
+          }
+        }
+        atomicMin(&s_bb[0], mnx);
+        atomicMin(&s_bb[1], mny);
+        atomicMax(&s_bb[2], mxx);
+        atomicMax(&s_bb[3], mxy);
+        __syncthreads();
+        if (tid == 0) {
+          sp.fb[part] = make_int4(s_fb[0], s_fb[1], s_fb[2], s_fb[3]);
+          sp.tb[part] = make_int4(s_bb[0], s_bb[1], s_bb[2], s_bb[3]);
+          if (kp == 0) sp.wb[ss] = make_int4(wx0, wy0, ww, wh);
+        }
       }
     }
     if constexpr (NH > 0) if (diag_on) {
@@ -1438,12 +1461,15 @@ __global__ __launch_bounds__(kThreads) void particle_kernel(BeamPtr<P> b, const 
                                            blockIdx.x, gridDim.y, blockIdx.y, win);
 }
 
-// The combine of a split particle pass (K parts per slice; one workgroup per
-// slice, after the pass): the slice's window as the sum of the K parts'
-// windows in part order, written to the source plane, its rectangle and
-// footprint, and the beam sums of the K parts in part order.  Parts that
-// added their windows with atomics (the batch's per-step launch) publish
-// through batch_publish_kernel instead.
+// The combine of a split particle pass (K parts per slice), after the pass.
+// Workgroups y < gridDim.y - 1 of a slice take 256 cells of its window each:
+// the sum of the K parts' windows in part order, written to the source plane.
+// The last one publishes the slice's rectangle and footprint from the parts'
+// boxes and the beam sums of the K parts in part order.  Parts that added
+// their windows with atomics (the batch's per-step launch) publish through
+// batch_publish_kernel instead.  Bound: launch latency; one workgroup per
+// slice for all of it, each thread adding 12 cells of K windows one after
+// the other, took 17.7 us at one slice and K = 4.
 template <class P, bool TAB>
 __global__ __launch_bounds__(kThreads) void split_combine_kernel(
     const int32_t* off, ParticleParams prm_arg, const ParticleParams* __restrict__ tab,
@@ -1452,62 +1478,51 @@ __global__ __launch_bounds__(kThreads) void split_combine_kernel(
   const ParticleParams& prm = slice_params<TAB, P>(prm_arg, tab);
   const int s = blockIdx.x;
   const int tid = threadIdx.x;
-  const int64_t ss = sp.own ? 0 : s;
-  __shared__ int s_bb[4];
-  __shared__ int s_fb[4];
-  if ((prm.stages & ST_DEP) && !sp.atomic_win) {
+  if (blockIdx.y + 1 < gridDim.y) {
+    const int4 wb = sp.wb[s];
+    const int k = blockIdx.y * kThreads + tid;
+    if (k >= wb.z * wb.w) return;
     const int ng = prm.dep.ngrid;
-    const int cap = prm.dep.window_cap;
+    const int64_t cap = prm.dep.window_cap;
+    const double2* parts = sp.win + static_cast<int64_t>(s) * K * cap + k;
+    double2 v = parts[0];
+    for (int q = 1; q < K; ++q) {
+      const double2 a = parts[q * cap];
+      v.x += a.x;
+      v.y += a.y;
+    }
+    T2 o;
+    o.x = static_cast<P>(v.x);
+    o.y = static_cast<P>(v.y);
     T2* src = static_cast<T2*>(prm.dep.src) + static_cast<int64_t>(s) * ng * ng;
-    const P scl = static_cast<P>(prm.dep.cur_over_npar[s] * prm.dep.scl_factor);
-    int wx0, wy0, ww, wh;
-    place_window(prm.dep.bbox[s], scl != P(0), ng, cap, wx0, wy0, ww, wh);
+    src[wb.x + k % wb.z + static_cast<int64_t>(wb.y + k / wb.z) * ng] = o;
+    return;
+  }
+  if ((prm.stages & ST_DEP) && tid < 64) {  // K <= 64: one wave
+    const int4 none = make_int4(0x7fffffff, 0x7fffffff, -1, -1);
+    const int64_t at = static_cast<int64_t>(s) * K + tid;
+    int4 f = tid < K ? sp.fb[at] : none, t = tid < K ? sp.tb[at] : none;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      f.x = min(f.x, __shfl_xor(f.x, o, 64));
+      f.y = min(f.y, __shfl_xor(f.y, o, 64));
+      f.z = max(f.z, __shfl_xor(f.z, o, 64));
+      f.w = max(f.w, __shfl_xor(f.w, o, 64));
+      t.x = min(t.x, __shfl_xor(t.x, o, 64));
+      t.y = min(t.y, __shfl_xor(t.y, o, 64));
+      t.z = max(t.z, __shfl_xor(t.z, o, 64));
+      t.w = max(t.w, __shfl_xor(t.w, o, 64));
+    }
     if (tid == 0) {
-      s_bb[0] = s_bb[1] = 0x7fffffff;
-      s_bb[2] = s_bb[3] = -1;
-      s_fb[0] = s_fb[1] = 0x7fffffff;
-      s_fb[2] = s_fb[3] = -1;
-      for (int q = 0; q < K; ++q) {
-        const int4 f = sp.fb[ss * K + q];
-        s_fb[0] = min(s_fb[0], f.x);
-        s_fb[1] = min(s_fb[1], f.y);
-        s_fb[2] = max(s_fb[2], f.z);
-        s_fb[3] = max(s_fb[3], f.w);
-      }
+      const int4 wb = sp.wb[s];
+      const int bb[4] = {t.x, t.y, t.z, t.w}, fb[4] = {f.x, f.y, f.z, f.w};
+      publish_boxes(prm, s, wb.x, wb.y, wb.z, wb.w, bb, fb);
     }
-    __syncthreads();
-    const double2* parts = sp.win + ss * K * cap;
-    int mnx = 0x7fffffff, mny = 0x7fffffff, mxx = -1, mxy = -1;
-    for (int k = tid; k < ww * wh; k += kThreads) {
-      const int cy = wy0 + k / ww, cx = wx0 + k % ww;
-      double2 v = parts[k];
-      for (int q = 1; q < K; ++q) {
-        const double2 a = parts[static_cast<int64_t>(q) * cap + k];
-        v.x += a.x;
-        v.y += a.y;
-      }
-      T2 o;
-      o.x = static_cast<P>(v.x);
-      o.y = static_cast<P>(v.y);
-      src[cx + static_cast<int64_t>(cy) * ng] = o;
-      if (v.x != 0.0 || v.y != 0.0) {
-        mnx = min(mnx, cx);
-        mny = min(mny, cy);
-        mxx = max(mxx, cx);
-        mxy = max(mxy, cy);
-      }
-    }
-    atomicMin(&s_bb[0], mnx);
-    atomicMin(&s_bb[1], mny);
-    atomicMax(&s_bb[2], mxx);
-    atomicMax(&s_bb[3], mxy);
-    __syncthreads();
-    if (tid == 0) publish_boxes(prm, s, wx0, wy0, ww, wh, s_bb, s_fb);
   }
   if (!(prm.stages & ST_DIAG)) return;
   const int nharm = prm.diag.nharm;
   const int nsum = 12 + 2 * nharm;
-  const double* parts = sp.red + ss * K * kRedStride;
+  const double* parts = sp.red + static_cast<int64_t>(s) * K * kRedStride;
   double* out = prm.diag.raw + static_cast<int64_t>(s) * G4H_BEAM_RAW(nharm);
   if (tid < nsum) {
     double v = 0.0;
@@ -1548,7 +1563,8 @@ __global__ void slice_kick_kernel(P* g, const int32_t* off, const double* dgamma
 }
 
 // Set-up of a split pass (K workgroups per slice), one workgroup per slice,
-// run before particle_kernel on the same stream: zero the cells the previous
+// run before particle_kernel on the same stream where the source planes are
+// not known to be clear or a footprint may be missing: zero the cells the previous
 // deposition left in the slice's source plane (the source rectangle), and on a
 // run's first deposition (no footprint yet) take the footprint of the
 // current positions into dep.bbox.  Doing the latter here rather than in each
@@ -1607,8 +1623,21 @@ __global__ void split_prepass_kernel(BeamPtr<P> b, const int32_t* off, ParticleP
 }
 
 // Workgroups per slice: a pass over few slices is split so that about two
-// workgroups per CU are in flight, keeping at least 8 iterations of the
-// particle loop per workgroup (or as pinned on the context).
+// workgroups per CU are in flight, keeping at least kSplitIters iterations of
+// the particle loop per workgroup (or as pinned on the context).  Below two
+// iterations the windows that a part clears and writes cost as much as the
+// particles; more workgroups than the target wait for LDS.  Step times by K
+// (us; * chosen):
+//   slices x particles, G          1    2    4     8    16     32    64
+//   1 x 8192, 151 FP64           143   99   73    60   55*     56    62
+//   1 x 16384, 255 MIXED         204  131   90    71   63      62*   66
+//   32 x 4096, 101 MIXED          66   55   48    44*  46      71
+//   64 x 8192, 151 FP64          164  117   93    86*  103    128   198
+//   128 x 4096, 128 MIXED         83   72   68*   86   112    178
+//   256 x 8192, 101 MIXED        116  103*  115   135  190    298   556
+constexpr int kSplitIters = 2;
+}  // namespace
+
 int split_of(Context* ctx, const Beam* b) {
   const int forced = ctx->tuner.forced[TUNE_SPLIT];
   if (forced >= 1) return std::min(forced, 64);
@@ -1620,26 +1649,35 @@ int split_of(Context* ctx, const Beam* b) {
   const int target = 2 * ctx->num_cus;
   if (b->nslice >= target) return 1;
   int k = (target + b->nslice - 1) / b->nslice;
-  k = std::min(k, b->max_slice_np / (8 * kThreads));
+  k = std::min(k, b->max_slice_np / (kSplitIters * kThreads));
   return std::max(1, std::min(k, 64));
 }
 
+namespace {
+// Parameters of a launch: by value, as a block already in device memory
+// (FP64; ParticleLaunch::d_prm), or a table with an entry per slice.
 template <class P, int NF, bool DEP, int NH, bool TAB>
 void launch_t(Context* ctx, Beam* b, const ParticleParams& p, BeamPtr<P> bp,
-              const ParticleParams* tab) {
+              const ParticleLaunch& how) {
   const size_t lds = DEP ? static_cast<size_t>(p.dep.window_cap) * sizeof(double2) : 0;
   const int K = split_of(ctx, b);
-  if (!tab && sizeof(P) == 8)
-    tab = static_cast<const ParticleParams*>(ctx->param_push(&p, sizeof(p)));
-  SplitScratch sp{nullptr, nullptr, nullptr, 0, 0};
+  const ParticleParams* tab = how.d_table ? how.d_table : how.d_prm;
+  const bool own = !tab && sizeof(P) == 8;
+  if (own) tab = static_cast<const ParticleParams*>(ctx->param_push(&p, sizeof(p)));
+  SplitScratch sp{};
   if (K > 1) {
     const size_t parts = static_cast<size_t>(b->nslice) * K;
     const size_t nwin = DEP ? parts * static_cast<size_t>(p.dep.window_cap) : 0;
+    const size_t nbox = 2 * parts + static_cast<size_t>(b->nslice);
     if (b->split_win.size() < nwin) b->split_win.alloc(ctx, nwin);
     if (b->split_red.size() < parts * kRedStride) b->split_red.alloc(ctx, parts * kRedStride);
-    if (b->split_fb.size() < parts) b->split_fb.alloc(ctx, parts);
-    sp = SplitScratch{b->split_win.get(), b->split_red.get(), b->split_fb.get(), 0, 0};
-    if (DEP) {
+    if (b->split_fb.size() < nbox) b->split_fb.alloc(ctx, nbox);
+    sp.win = b->split_win.get();
+    sp.red = b->split_red.get();
+    sp.fb = b->split_fb.get();
+    sp.tb = sp.fb + parts;
+    sp.wb = sp.tb + parts;
+    if (DEP && how.prepass) {
       ctx->launch(G4H_K_OTHER, [&] {
         hipLaunchKernelGGL((split_prepass_kernel<P, TAB>), dim3(b->nslice), dim3(256), 0,
                            ctx->stream, bp, b->off.get(), p, tab);
@@ -1651,41 +1689,42 @@ void launch_t(Context* ctx, Beam* b, const ParticleParams& p, BeamPtr<P> bp,
                        dim3(kThreads), lds, ctx->stream, bp, b->off.get(), p, tab, sp);
   });
   if (K > 1 && (DEP || NH > 0)) {
+    const int nwg = DEP ? (p.dep.window_cap + kThreads - 1) / kThreads : 0;
     ctx->launch(G4H_K_OTHER, [&] {
-      hipLaunchKernelGGL((split_combine_kernel<P, TAB>), dim3(b->nslice), dim3(kThreads), 0,
-                         ctx->stream, b->off.get(), p, tab, sp, K);
+      hipLaunchKernelGGL((split_combine_kernel<P, TAB>), dim3(b->nslice, nwg + 1), dim3(kThreads),
+                         0, ctx->stream, b->off.get(), p, tab, sp, K);
     });
   }
-  ctx->param_commit();
+  if (own) ctx->param_commit();
 }
 
 template <class P, int NF, bool DEP, bool TAB>
 void dispatch_nh(Context* ctx, Beam* b, const ParticleParams& p, BeamPtr<P> bp,
-                 const ParticleParams* tab) {
-  if (!(p.stages & ST_DIAG)) return launch_t<P, NF, DEP, 0, TAB>(ctx, b, p, bp, tab);
+                 const ParticleLaunch& how) {
+  if (!(p.stages & ST_DIAG)) return launch_t<P, NF, DEP, 0, TAB>(ctx, b, p, bp, how);
   const int nh = p.diag.nharm;
-  if (nh == 1) return launch_t<P, NF, DEP, 1, TAB>(ctx, b, p, bp, tab);
-  if (nh == 2) return launch_t<P, NF, DEP, 2, TAB>(ctx, b, p, bp, tab);
-  if (nh <= 4) return launch_t<P, NF, DEP, 4, TAB>(ctx, b, p, bp, tab);
-  return launch_t<P, NF, DEP, 8, TAB>(ctx, b, p, bp, tab);
+  if (nh == 1) return launch_t<P, NF, DEP, 1, TAB>(ctx, b, p, bp, how);
+  if (nh == 2) return launch_t<P, NF, DEP, 2, TAB>(ctx, b, p, bp, how);
+  if (nh <= 4) return launch_t<P, NF, DEP, 4, TAB>(ctx, b, p, bp, how);
+  return launch_t<P, NF, DEP, 8, TAB>(ctx, b, p, bp, how);
 }
 
 template <class P>
 void dispatch(Context* ctx, Beam* b, const ParticleParams& p, BeamPtr<P> bp,
-              const ParticleParams* tab) {
+              const ParticleLaunch& how) {
   const bool dep = (p.stages & ST_DEP) != 0;
   const bool single = !(p.stages & ST_PUSH) || p.push.nfield == 1;
-  if (tab) {
+  if (how.d_table) {
     require(single, "per-slice parameter tables serve single-field passes");
-    if (dep) return dispatch_nh<P, 1, true, true>(ctx, b, p, bp, tab);
-    return dispatch_nh<P, 1, false, true>(ctx, b, p, bp, tab);
+    if (dep) return dispatch_nh<P, 1, true, true>(ctx, b, p, bp, how);
+    return dispatch_nh<P, 1, false, true>(ctx, b, p, bp, how);
   }
   if (single) {
-    if (dep) return dispatch_nh<P, 1, true, false>(ctx, b, p, bp, nullptr);
-    return dispatch_nh<P, 1, false, false>(ctx, b, p, bp, nullptr);
+    if (dep) return dispatch_nh<P, 1, true, false>(ctx, b, p, bp, how);
+    return dispatch_nh<P, 1, false, false>(ctx, b, p, bp, how);
   }
-  if (dep) return dispatch_nh<P, 0, true, false>(ctx, b, p, bp, nullptr);
-  return dispatch_nh<P, 0, false, false>(ctx, b, p, bp, nullptr);
+  if (dep) return dispatch_nh<P, 0, true, false>(ctx, b, p, bp, how);
+  return dispatch_nh<P, 0, false, false>(ctx, b, p, bp, how);
 }
 
 // ---- batches of steady-state runs in one launch ----------------------------
@@ -1805,7 +1844,7 @@ __global__ __launch_bounds__(kThreads) void batch_step_particle_kernel(
   const ParticleParams& prm = tabk[pr.x];
   BeamPtr<P> b{static_cast<P*>(R.x),  static_cast<P*>(R.y), static_cast<P*>(R.px),
                static_cast<P*>(R.py), static_cast<P*>(R.g), R.th};
-  const SplitScratch sp{R.swin, R.sred, R.sfb, 1, 1};
+  const SplitScratch sp{R.swin, R.sred, R.sfb, nullptr, nullptr, 1, 1};
   particle_slice<P, 1, true, NH, kThreads, true>(b, R.off, prm, sp, R.slice, R.K, pr.y, lds);
 }
 
@@ -1911,8 +1950,7 @@ void launch_slice_kick(Context* ctx, Beam* b, const double* d_dgamma) {
   });
 }
 
-void launch_particle(Context* ctx, Beam* b, const ParticleParams& p,
-                     const ParticleParams* d_table) {
+void launch_particle(Context* ctx, Beam* b, const ParticleParams& p, const ParticleLaunch& how) {
   if (b->nslice <= 0) return;
   require(p.dep.window_cap * sizeof(double2) <= 96 * 1024 || !(p.stages & ST_DEP),
           "deposition window exceeds the LDS budget");
@@ -1921,11 +1959,11 @@ void launch_particle(Context* ctx, Beam* b, const ParticleParams& p,
   if (b->prec == G4H_FP64) {
     BeamPtr<double> bp{b->xd.get(), b->yd.get(), b->pxd.get(), b->pyd.get(), b->gd.get(),
                        b->theta.get()};
-    dispatch<double>(ctx, b, p, bp, d_table);
+    dispatch<double>(ctx, b, p, bp, how);
   } else {
     BeamPtr<float> bp{b->xf.get(), b->yf.get(), b->pxf.get(), b->pyf.get(), b->gf.get(),
                       b->theta.get()};
-    dispatch<float>(ctx, b, p, bp, d_table);
+    dispatch<float>(ctx, b, p, bp, how);
   }
 }
 
@@ -2087,7 +2125,7 @@ void diag_beam_raw_noalloc(Context* ctx, Beam* b, int nharm, double* raw) {
   auto* d_raw = reinterpret_cast<double*>(base + at);
   const size_t nraw = static_cast<size_t>(b->nslice) * G4H_BEAM_RAW(nharm);
   at += align256(nraw * sizeof(double));
-  SplitScratch sp{nullptr, nullptr, nullptr, 0, 0};
+  SplitScratch sp{};
   if (K > 1) {
     const size_t parts = static_cast<size_t>(b->nslice) * K;
     sp.red = reinterpret_cast<double*>(base + at);

@@ -48,6 +48,8 @@ struct g4h_run {
   double acc0 = 0.0;
   int end_first = 0, end_nrec = 0;
   double end_acc = 0.0;
+  bool deposited = false;        // this pass over the run has deposited
+  bool end_src_clear = false;    // Field::src_clear after the captured run
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   int field_generation = 0;  // of the field when captured
@@ -115,8 +117,16 @@ struct g4h_run {
       p.stages &= ~ST_T1;
       p.push.particle_ez = b->scez.get();
     }
-    launch_particle(ctx, b, p);
-    field_solve(f, src_on, out);
+    ParticleLaunch how;
+    // a captured run's first deposition always takes the pre-pass: a replay
+    // starts from whatever source and footprints the work before it left
+    how.prepass = source_needs_prepass(f, b) || (ctx->capturing && !deposited);
+    launch_particle(ctx, b, p, how);
+    if (src_on) {
+      source_deposited(f, b);
+      deposited = true;
+    }
+    field_solve(f, src_on, out, split_of(ctx, b) > 1);
     const Shifted z = slippage_host(f, st.slippage, cfg.sample, cfg.timerun, cfg.periodic);
     field_finish(f, z, out ? field_hist.get() + nrec * field_rec() : nullptr);
     if (out) {
@@ -236,6 +246,10 @@ g4h_status g4h_run_capture(g4h_run* r) {
   r->end_nrec = r->nrec;
   r->done = 0;
   r->nrec = 0;
+  r->deposited = false;
+  // a capture executes nothing: the source stays as the eager work left it
+  const bool src_clear = r->f->src_clear;
+  const uint64_t src_epoch = r->f->src_epoch;
   r->f->first = r->first0;
   r->f->accuslip = r->acc0;
   ctx->capturing = true;
@@ -250,6 +264,8 @@ g4h_status g4h_run_capture(g4h_run* r) {
     if (g) (void)hipGraphDestroy(g);
     ctx->capturing = false;
     ctx->arena = nullptr;
+    r->f->src_clear = src_clear;
+    r->f->src_epoch = src_epoch;
     r->done = static_cast<int>(r->steps.size());
     r->nrec = r->end_nrec;
     r->f->first = r->end_first;
@@ -261,6 +277,9 @@ g4h_status g4h_run_capture(g4h_run* r) {
   G4_HIP(hipStreamEndCapture(ctx->stream, &r->graph));
   G4_HIP(hipGraphInstantiate(&r->exec, r->graph, nullptr, nullptr, 0));
   r->field_generation = r->f->generation;
+  r->end_src_clear = r->f->src_clear;
+  r->f->src_clear = src_clear;
+  r->f->src_epoch = src_epoch;
   r->pez = r->b->pez_on ? r->b->pez.get() : nullptr;
   r->ef_generation = r->b->ef_generation;
   r->done = static_cast<int>(r->steps.size());
@@ -285,6 +304,10 @@ g4h_status g4h_run_replay(g4h_run* r) {
   r->ctx->activate();
   r->f->accuslip = r->acc0;
   G4_HIP(hipGraphLaunch(r->exec, r->ctx->stream));
+  if (r->deposited) {
+    source_deposited(r->f, r->b);
+    r->f->src_clear = r->end_src_clear;
+  }
   r->done = static_cast<int>(r->steps.size());
   r->nrec = r->end_nrec;
   r->f->first = r->end_first;
