@@ -42,6 +42,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "adi_lines.hpp"
@@ -765,21 +766,101 @@ __device__ __forceinline__ void glob_add(float* a, float v) {
   __hip_atomic_fetch_add((G4_GLOBAL float*)(a), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+// Extremes over the 64 lanes of the wave without LDS, as wave_total sums.
+template <class F>
+__device__ __forceinline__ double wave_fold(double v, F&& f) {
+  v = f(v, dpp_f64<0xB1>(v));
+  v = f(v, dpp_f64<0x4E>(v));
+  v = f(v, dpp_f64<0x141>(v));
+  v = f(v, dpp_f64<0x140>(v));
+  return f(f(lane_f64(v, 0), lane_f64(v, 16)), f(lane_f64(v, 32), lane_f64(v, 48)));
 }
-__device__ __forceinline__ double wave_min(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
-  return v;
+template <class F>
+__device__ __forceinline__ float wave_fold(float v, F&& f) {
+  auto dpp = [&](auto ctrl) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value,
+                                           0xf, 0xf, true));
+  };
+  v = f(v, dpp(std::integral_constant<int, 0xB1>{}));
+  v = f(v, dpp(std::integral_constant<int, 0x4E>{}));
+  v = f(v, dpp(std::integral_constant<int, 0x141>{}));
+  v = f(v, dpp(std::integral_constant<int, 0x140>{}));
+  auto lane = [&](int l) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+  };
+  return f(f(lane(0), lane(16)), f(lane(32), lane(48)));
 }
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-  return v;
+template <class F>
+__device__ __forceinline__ int wave_fold(int v, F&& f) {
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true));
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true));
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true));
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true));
+  return f(f(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+           f(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
+template <class T>
+__device__ __forceinline__ T wave_min(T v) {
+  return wave_fold(v, [](T p, T q) {
+    if constexpr (std::is_same_v<T, int>) return min(p, q);
+    else return fmin(p, q);
+  });
+}
+template <class T>
+__device__ __forceinline__ T wave_max(T v) {
+  return wave_fold(v, [](T p, T q) {
+    if constexpr (std::is_same_v<T, int>) return max(p, q);
+    else return fmax(p, q);
+  });
+}
+
+// Cells tid, tid + nt, ... of a rectangle w cells wide, without a division
+// per cell.  The ends of a workgroup's pass (one slice, or one part of it)
+// are latency alone: with the wave sums through shuffles, two divisions per
+// window cell and one LDS atomic per thread and bound they took 6 + 9 us; the
+// MIXED pass over 4096 x 16384 particles went from 1.21 to 1.15 ms with wave
+// folds and this walk, the FP64 one from 2.13 to 2.05 ms, one slice of 8192
+// particles (16 parts) from 28 to 17 us.
+struct CellWalk {
+  int x, y, dx, dy, w;
+  __device__ __forceinline__ CellWalk(int tid, int nt, int width) : w(max(width, 1)) {
+    y = tid / w;
+    x = tid - y * w;
+    dy = nt / w;
+    dx = nt - dy * w;
+  }
+  __device__ __forceinline__ void next() {
+    x += dx;
+    y += dy;
+    if (x >= w) {
+      x -= w;
+      ++y;
+    }
+  }
+};
+
+// Box (min x, min y, max x, max y) of the cells the threads of a workgroup
+// pass; the waves' boxes are folded into LDS box[0..3] (set empty before),
+// valid after the next barrier.  One atomic per wave and bound.
+struct CellBox {
+  int x0 = 0x7fffffff, y0 = 0x7fffffff, x1 = -1, y1 = -1;
+  __device__ __forceinline__ void add(int x, int y) {
+    x0 = min(x0, x);
+    y0 = min(y0, y);
+    x1 = max(x1, x);
+    y1 = max(y1, y);
+  }
+  __device__ __forceinline__ void fold(int* box) {
+    const int a = wave_min(x0), b = wave_min(y0), c = wave_max(x1), d = wave_max(y1);
+    if ((threadIdx.x & 63) == 0) {
+      atomicMin(&box[0], a);
+      atomicMin(&box[1], b);
+      atomicMax(&box[2], c);
+      atomicMax(&box[3], d);
+    }
+  }
+};
 
 // Per-thread partial sums of the beam diagnostics.  The energy and bunching
 // sums are FP64 in both modes.  The ten transverse moments are FP64 in FP64
@@ -1205,12 +1286,12 @@ __device__ __forceinline__ void particle_slice(BeamPtr<P> b, const int32_t* off,
     const int4 old = prm.dep.rect[s];
     const int ow = old.z - old.x, oh = old.w - old.y;
     if (K == 1 && ow > 0 && oh > 0) {
-      for (int k = tid; k < ow * oh; k += NT) {
-        const int cy = old.y + k / ow, cx = old.x + k % ow;
+      CellWalk at(tid, NT, ow);
+      for (int k = tid; k < ow * oh; k += NT, at.next()) {
         T2 z;
         z.x = 0;
         z.y = 0;
-        src[cx + static_cast<int64_t>(cy) * ng] = z;
+        src[old.x + at.x + static_cast<int64_t>(old.y + at.y) * ng] = z;
       }
     }
     for (int k = tid; k < ww * wh; k += NT) win[k] = make_double2(0.0, 0.0);
@@ -1296,14 +1377,13 @@ __device__ __forceinline__ void particle_slice(BeamPtr<P> b, const int32_t* off,
     for (int k = 0; k < NSUM; ++k) {
       if (k < nsum) {
         const double a = k < 2 ? ps.e[k] : (k < 12 ? static_cast<double>(ps.m[k - 2]) : ps.e[k - 10]);
-        const double v = wave_sum(a);
+        const double v = wave_total(a);
         if (lane == 0) s_red[wave][k] = v;
       }
     }
 #pragma unroll
     for (int k = 0; k < kNMinMax; ++k) {
-      const double m = static_cast<double>(ps.mm[k]);
-      const double v = (k & 1) ? wave_max(m) : wave_min(m);
+      const double v = static_cast<double>((k & 1) ? wave_max(ps.mm[k]) : wave_min(ps.mm[k]));
       if (lane == 0) s_red[wave][NSUM + k] = v;
     }
   }
@@ -1318,24 +1398,19 @@ __device__ __forceinline__ void particle_slice(BeamPtr<P> b, const int32_t* off,
     const int64_t part = ss * K + kp;
     if constexpr (DEP) if (dep_on) {
       if (sp.atomic_win) {
-        int mnx = 0x7fffffff, mny = 0x7fffffff, mxx = -1, mxy = -1;
-        for (int k = tid; k < ww * wh; k += NT) {
+        CellBox box;
+        CellWalk at(tid, NT, ww);
+        for (int k = tid; k < ww * wh; k += NT, at.next()) {
           const double2 v = win[k];
           if (v.x != 0.0 || v.y != 0.0) {
-            const int cy = wy0 + k / ww, cx = wx0 + k % ww;
+            const int cy = wy0 + at.y, cx = wx0 + at.x;
             P* a = reinterpret_cast<P*>(&src[cx + static_cast<int64_t>(cy) * ng]);
             glob_add(a, static_cast<P>(v.x));
             glob_add(a + 1, static_cast<P>(v.y));
-            mnx = min(mnx, cx);
-            mny = min(mny, cy);
-            mxx = max(mxx, cx);
-            mxy = max(mxy, cy);
+            box.add(cx, cy);
           }
         }
-        atomicMin(&s_bb[0], mnx);
-        atomicMin(&s_bb[1], mny);
-        atomicMax(&s_bb[2], mxx);
-        atomicMax(&s_bb[3], mxy);
+        box.fold(s_bb);
         __syncthreads();
         if (tid == 0) {
           int4 t = make_int4(s_bb[0], s_bb[1], s_bb[2], s_bb[3]);
@@ -1360,22 +1435,14 @@ __device__ __forceinline__ void particle_slice(BeamPtr<P> b, const int32_t* off,
         }
       } else {
         double2* w = sp.win + part * prm.dep.window_cap;
-        int mnx = 0x7fffffff, mny = 0x7fffffff, mxx = -1, mxy = -1;
-        for (int k = tid; k < ww * wh; k += NT) {
+        CellBox box;
+        CellWalk at(tid, NT, ww);
+        for (int k = tid; k < ww * wh; k += NT, at.next()) {
           const double2 v = win[k];
           w[k] = v;
-          if (v.x != 0.0 || v.y != 0.0) {
-            const int cy = wy0 + k / ww, cx = wx0 + k % ww;
-            mnx = min(mnx, cx);
-            mny = min(mny, cy);
-            mxx = max(mxx, cx);
-            mxy = max(mxy, cy);
-          }
+          if (v.x != 0.0 || v.y != 0.0) box.add(wx0 + at.x, wy0 + at.y);
         }
-        atomicMin(&s_bb[0], mnx);
-        atomicMin(&s_bb[1], mny);
-        atomicMax(&s_bb[2], mxx);
-        atomicMax(&s_bb[3], mxy);
+        box.fold(s_bb);
         __syncthreads();
         if (tid == 0) {
           sp.fb[part] = make_int4(s_fb[0], s_fb[1], s_fb[2], s_fb[3]);
@@ -1405,25 +1472,18 @@ __device__ __forceinline__ void particle_slice(BeamPtr<P> b, const int32_t* off,
     __syncthreads();
     // write the window with plain stores; its non-zero cells give the
     // footprint for the next step's window
-    int mnx = 0x7fffffff, mny = 0x7fffffff, mxx = -1, mxy = -1;
-    for (int k = tid; k < ww * wh; k += NT) {
-      const int cy = wy0 + k / ww, cx = wx0 + k % ww;
+    CellBox box;
+    CellWalk at(tid, NT, ww);
+    for (int k = tid; k < ww * wh; k += NT, at.next()) {
+      const int cy = wy0 + at.y, cx = wx0 + at.x;
       const double2 v = win[k];
       T2 o;
       o.x = static_cast<P>(v.x);
       o.y = static_cast<P>(v.y);
       src[cx + static_cast<int64_t>(cy) * ng] = o;
-      if (v.x != 0.0 || v.y != 0.0) {
-        mnx = min(mnx, cx);
-        mny = min(mny, cy);
-        mxx = max(mxx, cx);
-        mxy = max(mxy, cy);
-      }
+      if (v.x != 0.0 || v.y != 0.0) box.add(cx, cy);
     }
-    atomicMin(&s_bb[0], mnx);
-    atomicMin(&s_bb[1], mny);
-    atomicMax(&s_bb[2], mxx);
-    atomicMax(&s_bb[3], mxy);
+    box.fold(s_bb);
     __syncthreads();
     if (tid == 0) publish_boxes(prm, s, wx0, wy0, ww, wh, s_bb, s_fb);
   }
@@ -1629,12 +1689,12 @@ __global__ void split_prepass_kernel(BeamPtr<P> b, const int32_t* off, ParticleP
 // particles; more workgroups than the target wait for LDS.  Step times by K
 // (us; * chosen):
 //   slices x particles, G          1    2    4     8    16     32    64
-//   1 x 8192, 151 FP64           143   99   73    60   55*     56    62
-//   1 x 16384, 255 MIXED         204  131   90    71   63      62*   66
-//   32 x 4096, 101 MIXED          66   55   48    44*  46      71
-//   64 x 8192, 151 FP64          164  117   93    86*  103    128   198
-//   128 x 4096, 128 MIXED         83   72   68*   86   112    178
-//   256 x 8192, 101 MIXED        116  103*  115   135  190    298   556
+//   1 x 8192, 151 FP64           131   87   62    49   45*     45    51
+//   1 x 16384, 255 MIXED         194  120   79    60   51      51*   55
+//   32 x 4096, 101 MIXED          54   43   37    33*  34      45
+//   64 x 8192, 151 FP64          152  105   82    75*  82      95   137
+//   128 x 4096, 128 MIXED         72   61   57*   63   76     108
+//   256 x 8192, 101 MIXED        105   92*   95  103  125     171   316
 constexpr int kSplitIters = 2;
 }  // namespace
 
