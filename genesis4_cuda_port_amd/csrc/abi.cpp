@@ -83,8 +83,9 @@ void device_free(Context* ctx, void* p) {
     (void)hipFree(p);
 }
 
-const void* Context::param_push(const void* data, size_t bytes) {
+Context::ParamSlot Context::param_push(const void* data, size_t bytes) {
   require(bytes <= kParamBytes, "parameter block too large");
+  ParamSlot s;
   if (capturing) {
     require(arena && arena->used < arena->slots, "parameter arena of the capture is full");
     char* h = arena->host + static_cast<size_t>(arena->used) * kParamBytes;
@@ -92,7 +93,8 @@ const void* Context::param_push(const void* data, size_t bytes) {
     ++arena->used;
     std::memcpy(h, data, bytes);
     G4_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, stream));
-    return d;
+    s.dev = d;
+    return s;
   }
   if (!param_host) {
     void* h = nullptr;
@@ -114,15 +116,15 @@ const void* Context::param_push(const void* data, size_t bytes) {
   char* d = param_dev + static_cast<size_t>(k) * kParamBytes;
   std::memcpy(h, data, bytes);
   G4_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, stream));
-  param_last = k;
-  return d;
+  s.dev = d;
+  s.index = k;
+  return s;
 }
 
-void Context::param_commit() {
-  if (capturing || param_last < 0) return;
-  G4_HIP(hipEventRecord(param_ev[param_last], stream));
-  param_pending[param_last] = true;
-  param_last = -1;
+void Context::param_commit(const ParamSlot& s) {
+  if (s.index < 0) return;
+  G4_HIP(hipEventRecord(param_ev[s.index], stream));
+  param_pending[s.index] = true;
 }
 
 void Context::param_release() {
@@ -331,21 +333,21 @@ bool make_dep(DepParams& d, Field* f, Beam* b, const g4h_step& st, double delz) 
   return true;
 }
 
-// shared by g4h_apply_slippage and the fused run: the ring arithmetic; the
-// caller has the planes brought in zeroed (field_finish)
-Shifted slippage_host(Field* f, double slippage, double sample, int timerun, int periodic) {
+// shared by g4h_apply_slippage and the fused run: the ring arithmetic over n
+// slices; the caller has the planes brought in zeroed (field_finish)
+Shifted slippage_ring(int n, int& first, double& accuslip, double slippage, double sample,
+                      int timerun, int periodic) {
   Shifted z;
   if (!timerun) return z;
-  f->accuslip += slippage;
-  const int n = f->nslice;
+  accuslip += slippage;
   int direction = 1;
-  while (std::abs(f->accuslip) > (sample * 0.8)) {
-    direction = f->accuslip < 0 ? -1 : 1;
-    f->accuslip -= sample * direction;
-    int last = (f->first + n - 1) % n;
+  while (std::abs(accuslip) > (sample * 0.8)) {
+    direction = accuslip < 0 ? -1 : 1;
+    accuslip -= sample * direction;
+    int last = (first + n - 1) % n;
     if (direction < 0) last = (last + 1) % n;
-    f->first = last;
-    if (direction < 0) f->first = (last + 1) % n;
+    first = last;
+    if (direction < 0) first = (last + 1) % n;
     // a shift moves the planes brought in before it along with all others
     int& in = direction < 0 ? z.back : z.front;
     int& other = direction < 0 ? z.front : z.back;
@@ -941,7 +943,8 @@ g4h_status g4h_apply_slippage(g4h_context* ctx, g4h_field* f, double slippage, d
   G4_API_BEGIN
   require(ctx && f, "null argument");
   ctx->activate();
-  const Shifted z = slippage_host(f, slippage, sample, timerun, periodic);
+  const Shifted z = slippage_ring(f->nslice, f->first, f->accuslip, slippage, sample, timerun,
+                                  periodic);
   field_finish(f, z, nullptr);
   if (shifts) *shifts = z.shifts;
   G4_API_END

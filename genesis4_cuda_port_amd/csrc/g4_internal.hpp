@@ -182,18 +182,22 @@ struct Context {
   // Parameter blocks that kernels read through a pointer (rather than as
   // by-value arguments, which the compiler keeps live in scalar registers
   // and spills): staged through pinned host memory into a device ring.
-  // param_push copies a block into the next slot and returns its device
-  // address; param_commit marks the slot in use until the work enqueued so
-  // far on the stream has run.
-  static constexpr int kParamSlots = 64;
-  static constexpr size_t kParamBytes = 4096;
+  // param_push copies one or more blocks into the next slot; param_commit
+  // marks the slot in use until the work enqueued so far on the stream has
+  // run (nothing for an empty slot).
+  static constexpr int kParamSlots = 16;
+  static constexpr size_t kParamBytes = 16384;
+  struct ParamSlot {
+    const void* dev = nullptr;
+    int index = -1;
+  };
   char* param_host = nullptr;
   char* param_dev = nullptr;
   hipEvent_t param_ev[kParamSlots] = {};
   bool param_pending[kParamSlots] = {};
-  int param_next = 0, param_last = -1;
-  const void* param_push(const void* data, size_t bytes);
-  void param_commit();
+  int param_next = 0;
+  ParamSlot param_push(const void* data, size_t bytes);
+  void param_commit(const ParamSlot& slot);
   void param_release();
   // While capturing, blocks go to an arena that lives as long as the graph
   // (a replay reads them again): pinned host and device slots, filled in

@@ -316,7 +316,8 @@ double* field_partials(Field* f, int ntile);
 struct Shifted {
   int front = 0, back = 0, shifts = 0;
 };
-Shifted slippage_host(Field* f, double slippage, double sample, int timerun, int periodic);
+Shifted slippage_ring(int n, int& first, double& accuslip, double slippage, double sample,
+                      int timerun, int periodic);
 // Zero fill of the planes that slippage brought in and, with d_raw, the
 // record of the solve's field sums: raw[nslice*9] in logical order.
 void field_finish(Field* f, const Shifted& z, double* d_raw);

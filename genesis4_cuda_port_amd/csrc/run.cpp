@@ -80,56 +80,110 @@ struct g4h_run {
     ++nrec;
   }
 
-  void step(const g4h_step& st) {
+  // Particle-pass parameters of step st with the ring at `first` and the next
+  // record at rec.
+  struct Plan {
+    ParticleParams p;
+    bool src_on = false, out = false;
+  };
+  Plan plan_step(const g4h_step& st, int first, int rec) {
+    Plan q;
+    ParticleParams& p = q.p;
+    p = ParticleParams{};
     const double delz = st.delz;
     const double g0 = b->gamma_ref;
-    const bool out = cfg.record_diag && st.outstep && nrec < cap;
-    field_prepare_solver(f, delz);
-    ParticleParams p{};
+    q.out = cfg.record_diag && st.outstep && rec < cap;
     p.gamma0 = g0;
     p.stages = ST_T1 | ST_PUSH | ST_T2;
     p.t1 = make_trans(st, g0, delz * 0.5, false);
     p.t2 = make_trans(st, g0, delz * 0.5, true);
     Field* fl[1] = {f};
     make_push(p.push, st, g0, delz, fl, 1, nullptr);
+    p.push.f[0].first = first;
     p.push.particle_ez = b->pez_on ? b->pez.get() : nullptr;
     p.r56 = make_r56(st, g0, cfg.lambda0);
     if (p.r56 != 0.0) p.stages |= ST_R56;
-    const bool src_on = make_dep(p.dep, f, b, st, delz) && b->np > 0;
-    if (src_on) p.stages |= ST_DEP;
-    if (out) {
+    q.src_on = make_dep(p.dep, f, b, st, delz) && b->np > 0;
+    if (q.src_on) p.stages |= ST_DEP;
+    if (q.out) {
       p.stages |= ST_DIAG;
-      p.diag.raw = beam_hist.get() + nrec * beam_rec();
+      p.diag.raw = beam_hist.get() + rec * beam_rec();
       p.diag.nharm = cfg.nharm;
     }
+    return q;
+  }
+
+  // Steps [k0, k1).  Their parameters are planned ahead (the ring moves by
+  // host arithmetic alone) and, in FP64, uploaded as many at a time as a
+  // parameter slot holds: one copy of 4.5 us on the stream per dozen steps
+  // instead of one per step (MIXED passes them by value).
+  void steps_run(int k0, int k1) {
+    constexpr int kChunk = static_cast<int>(Context::kParamBytes / sizeof(ParticleParams));
+    std::vector<Plan> plan;
+    std::vector<ParticleParams> blocks;
+    while (k0 < k1) {
+      const int n = std::min(kChunk, k1 - k0);
+      plan.clear();
+      blocks.clear();
+      int first = f->first, rec = nrec;
+      double acc = f->accuslip;
+      for (int i = 0; i < n; ++i) {
+        const g4h_step& st = steps[static_cast<size_t>(k0 + i)];
+        plan.push_back(plan_step(st, first, rec));
+        if (plan.back().out) ++rec;
+        (void)slippage_ring(f->nslice, first, acc, st.slippage, cfg.sample, cfg.timerun,
+                            cfg.periodic);
+      }
+      // with space charge the pass is two, and reads the field it computes
+      if (b->ef.nz > 0)
+        for (Plan& q : plan) q.p.push.particle_ez = b->scez.get();
+      for (const Plan& q : plan) {
+        blocks.push_back(q.p);
+        if (b->ef.nz > 0) blocks.back().stages &= ~ST_T1;
+      }
+      Context::ParamSlot slot;
+      if (b->prec == G4H_FP64)
+        slot = ctx->param_push(blocks.data(), blocks.size() * sizeof(ParticleParams));
+      const auto* dev = static_cast<const ParticleParams*>(slot.dev);
+      for (int i = 0; i < n; ++i, ++done)
+        step(steps[static_cast<size_t>(k0 + i)], plan[static_cast<size_t>(i)],
+             blocks[static_cast<size_t>(i)], dev ? dev + i : nullptr);
+      ctx->param_commit(slot);
+      k0 += n;
+    }
+  }
+
+  void step(const g4h_step& st, const Plan& q, const ParticleParams& p,
+            const ParticleParams* d_prm) {
+    field_prepare_solver(f, st.delz);
     if (b->ef.nz > 0) {
       // BeamSolverCUDA::advance takes the short-range field from the
       // positions after the first transverse half step (Beam.cpp:123-125,
       // BeamSolverCUDA.cpp:523-547): that half step, the field, then the
       // rest of the pass with the field as its per-particle term
       ParticleParams p1{};
-      p1.gamma0 = g0;
+      p1.gamma0 = p.gamma0;
       p1.stages = ST_T1;
       p1.t1 = p.t1;
       launch_particle(ctx, b, p1);
-      launch_space_charge(ctx, b, g0 * g0 / (1.0 + st.aw * st.aw), nullptr,
+      launch_space_charge(ctx, b, p.gamma0 * p.gamma0 / (1.0 + st.aw * st.aw), nullptr,
                           b->pez_on ? b->pez.get() : nullptr);
-      p.stages &= ~ST_T1;
-      p.push.particle_ez = b->scez.get();
     }
     ParticleLaunch how;
+    how.d_prm = d_prm;
     // a captured run's first deposition always takes the pre-pass: a replay
     // starts from whatever source and footprints the work before it left
     how.prepass = source_needs_prepass(f, b) || (ctx->capturing && !deposited);
     launch_particle(ctx, b, p, how);
-    if (src_on) {
+    if (q.src_on) {
       source_deposited(f, b);
       deposited = true;
     }
-    field_solve(f, src_on, out, split_of(ctx, b) > 1);
-    const Shifted z = slippage_host(f, st.slippage, cfg.sample, cfg.timerun, cfg.periodic);
-    field_finish(f, z, out ? field_hist.get() + nrec * field_rec() : nullptr);
-    if (out) {
+    field_solve(f, q.src_on, q.out, split_of(ctx, b) > 1);
+    const Shifted z = slippage_ring(f->nslice, f->first, f->accuslip, st.slippage, cfg.sample,
+                                    cfg.timerun, cfg.periodic);
+    field_finish(f, z, q.out ? field_hist.get() + nrec * field_rec() : nullptr);
+    if (q.out) {
       if (b->ef.nz > 0 && sc_hist.size() >= static_cast<size_t>(nrec + 1) * b->nslice)
         G4_HIP(hipMemcpyAsync(sc_hist.get() + static_cast<size_t>(nrec) * b->nslice,
                               b->scrms.get(), sizeof(double) * b->nslice,
@@ -200,7 +254,7 @@ g4h_status g4h_run_advance(g4h_run* r, int nsteps, int* done) {
   require(nsteps >= 0, "nsteps must be >= 0");
   r->ctx->activate();
   const int end = std::min<int>(static_cast<int>(r->steps.size()), r->done + nsteps);
-  for (; r->done < end; ++r->done) r->step(r->steps[r->done]);
+  r->steps_run(r->done, end);
   if (done) *done = r->done;
   G4_API_END
 }
@@ -230,9 +284,12 @@ g4h_status g4h_run_capture(g4h_run* r) {
   }
   G4_HIP(hipStreamSynchronize(ctx->stream));
   ctx->tune_settle();
-  if (r->b->prec == G4H_FP64) {  // one parameter block per particle launch
-    // one parameter block per particle launch: two per step with space charge
-    const int slots = static_cast<int>(r->steps.size()) * (r->b->ef.nz > 0 ? 2 : 1) + 1;
+  if (r->b->prec == G4H_FP64) {
+    // parameter slots: the initial record, the steps' chunks, and with space
+    // charge each step's first half
+    constexpr size_t kChunk = Context::kParamBytes / sizeof(ParticleParams);
+    const size_t ns = r->steps.size();
+    const int slots = static_cast<int>(2 + ns / kChunk + (r->b->ef.nz > 0 ? ns : 0));
     void* h = nullptr;
     void* d = nullptr;
     G4_HIP(hipHostMalloc(&h, static_cast<size_t>(slots) * Context::kParamBytes, hipHostMallocDefault));
@@ -257,7 +314,7 @@ g4h_status g4h_run_capture(g4h_run* r) {
   G4_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
   try {
     r->record_initial();
-    for (const g4h_step& st : r->steps) r->step(st);
+    r->steps_run(0, static_cast<int>(r->steps.size()));
   } catch (...) {
     hipGraph_t g = nullptr;
     (void)hipStreamEndCapture(ctx->stream, &g);
