@@ -278,15 +278,15 @@ __device__ __forceinline__ void seg_x(const typename A2<P>::T* u, typename A2<P>
 // y sweep of columns 16 blk .. of one plane from the x sweep's output `in`;
 // every thread of the workgroup takes part.  ends: LDS [2][16][16]; with
 // STATS the block's field sums go to part[0..6] and the centre cell to
-// centre[0..1] (red: LDS [4][8]).  sclear: the source plane sp again, whose
-// cells this block read are then set to zero (the step's last reader of the
-// source clears it for the next deposition), or nullptr.
-template <class P, int K, bool STATS>
+// centre[0..1] (red: LDS [4][8]).  With CLEAR the source cells this block read
+// are then set to zero (the step's last reader of the source clears it for
+// the next deposition); as a run-time switch it took registers that K = 16
+// does not have (467 -> 542 us on 2048 planes without statistics).
+template <class P, int K, bool STATS, bool CLEAR>
 __device__ __forceinline__ void seg_y(const typename A2<P>::T* in, typename A2<P>::T* u, int G,
                                       double cs, const double2* tab,
                                       const typename A2<P>::T* sp, int4 rc, int blk,
-                                      double2* ends, double* red, double* part, double* centre,
-                                      typename A2<P>::T* sclear) {
+                                      double2* ends, double* red, double* part, double* centre) {
   using T2 = typename A2<P>::T;
   constexpr int E = sizeof(T2);
   const int c = threadIdx.x % kSegLines, t = threadIdx.x / kSegLines;
@@ -374,14 +374,13 @@ __device__ __forceinline__ void seg_y(const typename A2<P>::T* in, typename A2<P
       }
     }
   }
-  if (sclear && src) {
-    const Rsrc rw = plane_rsrc(sclear, G, E);
+  if (CLEAR && src) {
     T2 z;
     z.x = 0;
     z.y = 0;
 #pragma unroll
     for (int j = 0; j < K; ++j)
-      bstore<0>(rw, cell_off(scol && row0 + j >= rc.y && row0 + j < rc.w, row0 + j, col, G, E), z);
+      bstore<0>(rs, cell_off(scol && row0 + j >= rc.y && row0 + j < rc.w, row0 + j, col, G, E), z);
   }
   if constexpr (STATS) {
     const double dx = col + shift;

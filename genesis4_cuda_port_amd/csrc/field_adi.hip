@@ -415,11 +415,11 @@ __global__ __launch_bounds__(adi::kSegThreads, K > 10 ? 3 : 4) void adi_x_seg_ke
 // ... and the y sweep, with the block's field sums in the layout of the
 // wave-per-block variants (partials[(p * nblk + b) * 8 + k], centres at the
 // tail).
-template <class P, int K, bool STATS>
+template <class P, int K, bool STATS, bool CLEAR>
 __global__ __launch_bounds__(adi::kSegThreads, K > 10 ? 3 : 4) void adi_y_seg_kernel(
     typename A2<P>::T* u, const typename A2<P>::T* ustar, int nslice, int nblk, int G, double cs,
     const double2* __restrict__ tab, const typename A2<P>::T* src, const int4* rect, int first,
-    int add_src, int clear_src, double* partials) {
+    int add_src, double* partials) {
   using T2 = typename A2<P>::T;
   extern __shared__ double2 lds[];
   const SegBlock b = seg_block(nblk);
@@ -438,9 +438,8 @@ __global__ __launch_bounds__(adi::kSegThreads, K > 10 ? 3 : 4) void adi_y_seg_ke
   double* red = reinterpret_cast<double*>(ends + 2 * adi::kSegs * adi::kSegLines);
   double* part = STATS ? partials + (static_cast<int64_t>(b.p) * nblk + b.blk) * 8 : nullptr;
   double* centre = STATS ? partials + static_cast<int64_t>(nslice) * nblk * 8 + 2 * b.p : nullptr;
-  adi::seg_y<P, K, STATS>(ustar + b.p * plane, u + b.p * plane, G, cs, lds, sp, rc, b.blk, ends,
-                          red, part, centre,
-                          clear_src ? const_cast<T2*>(sp) : nullptr);
+  adi::seg_y<P, K, STATS, CLEAR>(ustar + b.p * plane, u + b.p * plane, G, cs, lds, sp, rc, b.blk,
+                                 ends, red, part, centre);
 }
 
 // The segmented sweeps of every run of a batch in one launch: workgroup b
@@ -473,9 +472,9 @@ __global__ __launch_bounds__(adi::kSegThreads, 3) void adi_x_seg_batch_kernel(
   });
 }
 
-template <class P, bool STATS>
+template <class P, bool STATS, bool CLEAR>
 __global__ __launch_bounds__(adi::kSegThreads, 3) void adi_y_seg_batch_kernel(
-    const BatchSegDesc* __restrict__ blocks, int k, int add_src, int clear_src) {
+    const BatchSegDesc* __restrict__ blocks, int k, int add_src) {
   using T2 = typename A2<P>::T;
   extern __shared__ double2 lds[];
   const BatchSegDesc D = blocks[blockIdx.x];
@@ -493,7 +492,6 @@ __global__ __launch_bounds__(adi::kSegThreads, 3) void adi_y_seg_batch_kernel(
   }
   const T2* in = static_cast<const T2*>(D.ustar) + D.slice * plane;
   T2* out = static_cast<T2*>(D.u) + D.slice * plane;
-  T2* clr = clear_src && sp ? const_cast<T2*>(sp) : nullptr;
   double2* ends = lds + ntab;
   double* red = reinterpret_cast<double*>(ends + 2 * adi::kSegs * adi::kSegLines);
   double* part =
@@ -502,8 +500,8 @@ __global__ __launch_bounds__(adi::kSegThreads, 3) void adi_y_seg_batch_kernel(
       STATS ? D.partials + static_cast<int64_t>(D.nrun) * D.nblk * 8 + 2 * D.slice : nullptr;
   const double cs = D.cs[k];
   adi::with_seg_len(G, [&](auto len) {
-    adi::seg_y<P, decltype(len)::value, STATS>(in, out, G, cs, lds, sp, rc, D.blk, ends, red, part,
-                                               centre, clr);
+    adi::seg_y<P, decltype(len)::value, STATS, CLEAR>(in, out, G, cs, lds, sp, rc, D.blk, ends,
+                                                      red, part, centre);
   });
 }
 
@@ -571,7 +569,6 @@ void adi_step(Field* f, bool source_on, bool stats, bool clear) {
     T2* ustar = static_cast<T2*>(adi_ustar(f));
     const double2* tab = f->adi_c + 3 * G;
     const dim3 block(adi::kSegThreads);
-    const int clr = clear ? 1 : 0;
     const dim3 grid(static_cast<unsigned>((f->nslice + 7) / 8) * 8 * nblk);
     adi::with_seg_len(G, [&](auto len) {
       constexpr int K = decltype(len)::value;
@@ -580,16 +577,17 @@ void adi_step(Field* f, bool source_on, bool stats, bool clear) {
                            f->ctx->stream, u, ustar, f->nslice, nblk, G, cs, tab, src,
                            f->src_rect.get(), f->first, add);
       });
-      f->ctx->launch(G4H_K_ADI_Y, [&] {
-        if (stats)
-          hipLaunchKernelGGL((adi_y_seg_kernel<P, K, true>), grid, block, adi::seg_lds_y(K),
-                             f->ctx->stream, u, ustar, f->nslice, nblk, G, cs, tab, src,
-                             f->src_rect.get(), f->first, add, clr, partials);
-        else
-          hipLaunchKernelGGL((adi_y_seg_kernel<P, K, false>), grid, block, adi::seg_lds_y(K),
-                             f->ctx->stream, u, ustar, f->nslice, nblk, G, cs, tab, src,
-                             f->src_rect.get(), f->first, add, clr, partials);
-      });
+      auto y = [&](auto kern) {
+        f->ctx->launch(G4H_K_ADI_Y, [&] {
+          hipLaunchKernelGGL(kern, grid, block, adi::seg_lds_y(K), f->ctx->stream, u, ustar,
+                             f->nslice, nblk, G, cs, tab, src, f->src_rect.get(), f->first, add,
+                             partials);
+        });
+      };
+      if (stats)
+        y(clear ? adi_y_seg_kernel<P, K, true, true> : adi_y_seg_kernel<P, K, true, false>);
+      else
+        y(clear ? adi_y_seg_kernel<P, K, false, true> : adi_y_seg_kernel<P, K, false, false>);
     });
     if (clear) f->src_clear = true;
     return;
@@ -652,7 +650,7 @@ void launch_batch_adi_step(Context* ctx, g4h_precision prec, const BatchSegDesc*
   if (nblocks <= 0) return;
   require(gmax <= adi::kSegMaxGrid, "segmented sweeps: ngrid above 256");
   const size_t ldsx = adi::seg_lds_x(adi::seg_len(gmax)), ldsy = adi::seg_lds_y(adi::seg_len(gmax));
-  const int src = add_src ? 1 : 0, clr = clear_src ? 1 : 0;
+  const int src = add_src ? 1 : 0;
   ctx->launch(G4H_K_ADI_X, [&] {
     if (prec == G4H_FP64)
       hipLaunchKernelGGL(adi_x_seg_batch_kernel<double>, dim3(nblocks), dim3(adi::kSegThreads),
@@ -664,20 +662,21 @@ void launch_batch_adi_step(Context* ctx, g4h_precision prec, const BatchSegDesc*
   auto y = [&](auto kern) {
     ctx->launch(G4H_K_ADI_Y, [&] {
       hipLaunchKernelGGL(kern, dim3(nblocks), dim3(adi::kSegThreads), ldsy, ctx->stream,
-                         d_blocks, k, src, clr);
+                         d_blocks, k, src);
     });
   };
-  if (prec == G4H_FP64) {
+  auto pick = [&](auto p) {
+    using P = decltype(p);
     if (stats)
-      y(adi_y_seg_batch_kernel<double, true>);
+      y(clear_src ? adi_y_seg_batch_kernel<P, true, true> : adi_y_seg_batch_kernel<P, true, false>);
     else
-      y(adi_y_seg_batch_kernel<double, false>);
-  } else {
-    if (stats)
-      y(adi_y_seg_batch_kernel<float, true>);
-    else
-      y(adi_y_seg_batch_kernel<float, false>);
-  }
+      y(clear_src ? adi_y_seg_batch_kernel<P, false, true>
+                  : adi_y_seg_batch_kernel<P, false, false>);
+  };
+  if (prec == G4H_FP64)
+    pick(double{});
+  else
+    pick(float{});
 }
 
 void launch_batch_field_records(Context* ctx, const BatchRunDesc* d_runs, int nruns, int r) {
