@@ -17,9 +17,11 @@
 //
 // Transforms: power-of-two sizes use register-resident radix-2 transforms
 // (forward DIF, inverse DIT, multipliers in bit-reversed order); other sizes
-// use a direct DFT in LDS.  With the source filter on (non-separable), the filtered
+// up to 512 step their lines by convolution through such transforms, larger
+// ones and the source filter use a direct DFT in LDS.  With the source filter on (non-separable), the filtered
 // source T = 2 IFFT2(filt FFT2(S))/G^2 is built in a work plane first
 // (FWD rows, FWD*filt*INV columns, INV rows) and added in place of 2S.
+#include "buffer_access.hpp"
 #include "fft_regs.hpp"
 #include "kernels.hpp"
 
@@ -607,7 +609,244 @@ __global__ void gather_source_kernel(const typename C2<P>::T* src, const int4* r
 }
 
 // ---------------------------------------------------------------------------
-// Other sizes N with the propagator: convolution through power-of-two
+// Other sizes N < 256 with the propagator: convolution through pairs of
+// Q-point transforms, Q the power of two above N.  One line's step
+// IDFT_N(P . DFT_N(u)) is the circular convolution of u with h = IDFT_N(P).
+// With g_k = h_(k mod N), |k| < N, wrapped onto M = 2Q >= 2N - 1 points, a
+// circular convolution of M points gives the line's N values at 0 .. N - 1.
+// u is zero beyond Q, so the M-point spectrum falls into two Q-point ones,
+//   X_(2m) = DFT_Q(u),  X_(2m+1) = DFT_Q(u_n w_n),  w_n = exp(-2 pi i n / M),
+// and the first Q results into two Q-point inverse transforms,
+//   y_n = IDFT_Q(H_(2m) X_(2m))_n + conj(w_n) IDFT_Q(H_(2m+1) X_(2m+1))_n,
+// with H = DFT_M(g) / M: four Q-point register transforms instead of two
+// M-point ones whose upper half is zeros on the way in and dropped on the way
+// out.  Registers hold two Q-point lines, the transpose buffers one.
+// Bound: VALU and LDS (four 256-point transforms where a power-of-two line has
+// two); the FP64 column pass reaches 4.0 TB/s.  Addresses are 32-bit buffer
+// offsets: 64-bit ones, live from the loads to the stores, took 205 registers
+// where the MIXED passes now take 88 and 115.  Column + row pass, two M-point
+// transforms -> this:
+//   1024 planes, N = 151, MIXED   257 + 187 us -> 162 + 142 us
+//   256 planes, N = 255, FP64     495 + 348 us -> 134 + 209 us
+// N from 257 (two lines of 512 points, 256 registers in FP64) stays with the
+// M-point transforms below.
+// ---------------------------------------------------------------------------
+template <class P, int Q>
+struct HalfCfg {
+  using S = fftr::Shape<Q>;
+  static constexpr int kWaves = 4;
+  static constexpr int kThreads = 64 * kWaves;
+  static constexpr int TW = kThreads / S::L;  // columns per column-pass tile
+  static constexpr int kBuf = kWaves * S::LPW * S::BUF;
+  // transposes take real and imaginary parts in turn (fftr::xpose): half the
+  // buffer, so that LDS does not limit the workgroups per CU
+  using B = P;
+  static constexpr int kMinWaves = S::L == 1 ? 1 : (sizeof(P) == 8 ? 3 : 4);  // per SIMD
+};
+
+// The step of one line held as v (natural layout): tw the four-step
+// twiddles, mu the even then the odd multipliers in pi order, wn[Q].
+template <class T2, int Q, int STRIDE, bool BLOCK, class B>
+__device__ __forceinline__ void half_line_step(T2 (&v)[fftr::Shape<Q>::R], int t, const T2* tw,
+                                               const T2* mu, const T2* wn, B* buf) {
+  using S = fftr::Shape<Q>;
+  constexpr int R = S::R, L = S::L;
+  // The stages stay in program order (table reads four at a time): overlapped
+  // by the scheduler they took 205 registers in MIXED and spilled in FP64.
+  auto fence = [](auto ic) {
+    if constexpr (decltype(ic)::value % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+  };
+  T2 a[R];
+  fftr::static_for<0, R>([&](auto ic) { a[decltype(ic)::value] = v[decltype(ic)::value]; });
+  __builtin_amdgcn_sched_barrier(0);
+  fftr::forward<T2, Q, STRIDE, BLOCK>(a, t, tw, buf);
+  __builtin_amdgcn_sched_barrier(0);
+  fftr::static_for<0, R>([&](auto ic) {
+    constexpr int q = decltype(ic)::value;
+    a[q] = fftr::cmul(a[q], mu[q * L + t]);
+    fence(ic);
+  });
+  fftr::inverse<T2, Q, STRIDE, BLOCK>(a, t, tw, buf);
+  __builtin_amdgcn_sched_barrier(0);
+  fftr::static_for<0, R>([&](auto ic) {
+    constexpr int r = decltype(ic)::value;
+    v[r] = fftr::cmul(v[r], wn[t + L * r]);
+    fence(ic);
+  });
+  if constexpr (BLOCK) __syncthreads();  // the transpose buffer is used again
+  fftr::forward<T2, Q, STRIDE, BLOCK>(v, t, tw, buf);
+  __builtin_amdgcn_sched_barrier(0);
+  fftr::static_for<0, R>([&](auto ic) {
+    constexpr int q = decltype(ic)::value;
+    v[q] = fftr::cmul(v[q], mu[Q + q * L + t]);
+    fence(ic);
+  });
+  fftr::inverse<T2, Q, STRIDE, BLOCK>(v, t, tw, buf);
+  __builtin_amdgcn_sched_barrier(0);
+  fftr::static_for<0, R>([&](auto ic) {
+    constexpr int r = decltype(ic)::value;
+    v[r] = fftr::cadd(a[r], fftr::cmulc(v[r], wn[t + L * r]));
+    fence(ic);
+  });
+}
+
+template <class P, int Q>
+__global__ __launch_bounds__((HalfCfg<P, Q>::kThreads), (HalfCfg<P, Q>::kMinWaves)) void
+fft_rows_half_kernel(typename C2<P>::T* u, int64_t nrows, int N, const double2* tw_d,
+                     const double2* mult_d) {
+  using T2 = typename C2<P>::T;
+  using S = fftr::Shape<Q>;
+  using C = HalfCfg<P, Q>;
+  constexpr int R = S::R, L = S::L, E = sizeof(T2);
+  __shared__ T2 tw[Q];
+  __shared__ T2 wn[Q];
+  __shared__ T2 mu[2 * Q];
+  __shared__ typename C::B buf[C::kBuf];
+  load_table(tw, tw_d, Q);
+  load_table(wn, tw_d + Q, Q);
+  load_table(mu, mult_d, 2 * Q);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane / L, t = lane % L;
+  typename C::B* lbuf = buf + (wave * S::LPW + g) * S::BUF;
+  const int64_t nwaves = static_cast<int64_t>(gridDim.x) * C::kWaves;
+  for (int64_t grp = blockIdx.x * static_cast<int64_t>(C::kWaves) + wave; grp * S::LPW < nrows;
+       grp += nwaves) {
+    // the wave's lines as one buffer: lines past the last are out of range
+    const int64_t line0 = grp * S::LPW;
+    const int nl = static_cast<int>(min<int64_t>(S::LPW, nrows - line0));
+    const Rsrc ru = range_rsrc(u + line0 * N, nl * N * E);
+    const uint32_t o0 = static_cast<uint32_t>(g * N + t) * E;
+    T2 v[R];
+    fftr::static_for<0, R>([&](auto ic) {
+      constexpr int r = decltype(ic)::value;
+      v[r] = bload<0, T2>(ru, t + L * r < N ? o0 + L * r * E : kOut);
+    });
+    half_line_step<T2, Q, 1, false>(v, t, tw, mu, wn, lbuf);
+    fftr::static_for<0, R>([&](auto ic) {
+      constexpr int r = decltype(ic)::value;
+      bstore<0>(ru, t + L * r < N ? o0 + L * r * E : kOut, v[r]);
+    });
+  }
+}
+
+// Column pass: tiles of TW adjacent columns as in fft_cols_reg_kernel (thread
+// (t, column tid % TW) holds rows t + L r).  The tiles of a plane share an
+// XCD (workgroups go to the eight XCDs round robin) and plain accesses:
+// with N odd every row segment cuts cache lines that the neighbouring tiles
+// complete in L2.
+// WORK: the filtered source of the work plane is added (a variant of its own:
+// beside the other source it doubled the registers).
+template <class P, int Q, bool WORK>
+__global__ __launch_bounds__((HalfCfg<P, Q>::kThreads), (HalfCfg<P, Q>::kMinWaves)) void
+fft_cols_half_kernel(typename C2<P>::T* u, int nslice, int N, const double2* tw_d,
+                     const double2* mult_d, typename C2<P>::T* src, const int4* rect, int first,
+                     int add_src, int clear_src, const double2* work, double* partials) {
+  using T2 = typename C2<P>::T;
+  using S = fftr::Shape<Q>;
+  using C = HalfCfg<P, Q>;
+  constexpr int R = S::R, L = S::L, TW = C::TW, E = sizeof(T2);
+  __shared__ T2 tw[Q];
+  __shared__ T2 wn[Q];
+  __shared__ T2 mu[2 * Q];
+  __shared__ typename C::B buf[C::kBuf];
+  __shared__ double red[C::kWaves][8];
+  const int ntile = (N + TW - 1) / TW;
+  const int p = (blockIdx.x >> 3) / ntile * 8 + (blockIdx.x & 7);
+  const int tile = (blockIdx.x >> 3) % ntile;
+  if (p >= nslice) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int t = static_cast<int>(threadIdx.x) / TW;
+  const int cslot = static_cast<int>(threadIdx.x) % TW;
+  const int col = tile * TW + cslot;
+  // rows past the last are beyond the plane, columns past it at kOut
+  const Rsrc ru = plane_rsrc(u + static_cast<int64_t>(p) * N * N, N, E);
+  const uint32_t o0 = cell_off(col < N, t, col, N, E);
+  const uint32_t ostep = static_cast<uint32_t>(L) * N * E;
+  T2 v[R];
+  fftr::static_for<0, R>([&](auto ic) {
+    constexpr int r = decltype(ic)::value;
+    v[r] = bload<0, T2>(ru, o0 + r * ostep);
+  });
+  load_table(tw, tw_d, Q);
+  load_table(wn, tw_d + Q, Q);
+  load_table(mu, mult_d, 2 * Q);
+  __syncthreads();
+  half_line_step<T2, Q, TW, true>(v, t, tw, mu, wn, buf + cslot);
+  // the addresses anew: kept from the loads they would hold R registers
+  uint32_t o1 = o0, ostep1 = ostep;
+  asm volatile("" : "+v"(o1), "+s"(ostep1));
+
+  const int s = ((p - first) % nslice + nslice) % nslice;  // beam slice of this ring plane
+  int4 rc = make_int4(0, 0, 0, 0);
+  if (!WORK && add_src == 1) rc = rect[s];
+  const bool src_on =
+      !WORK && add_src == 1 && tile * TW < rc.z && (tile + 1) * TW > rc.x;  // uniform
+  if (src_on) {
+    const Rsrc rs = plane_rsrc(src + static_cast<int64_t>(s) * N * N, N, E);
+    const bool scol = col >= rc.x && col < rc.z;
+    fftr::static_for<0, R>([&](auto ic) {
+      constexpr int r = decltype(ic)::value;
+      const int row = t + L * r;
+      const uint32_t o = scol && row >= rc.y && row < rc.w ? o1 + r * ostep1 : kOut;
+      const T2 sv = bload<0, T2>(rs, o);
+      v[r].x += P(2) * sv.x;
+      v[r].y += P(2) * sv.y;
+      if (clear_src) bstore<0>(rs, o, T2{});
+      if constexpr (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+  if constexpr (WORK) {
+    const Rsrc rw = plane_rsrc(work + static_cast<int64_t>(p) * N * N, N, 16);
+    fftr::static_for<0, R>([&](auto ic) {
+      constexpr int r = decltype(ic)::value;
+      const double2 wv = bload<0, double2>(rw, cell_off(col < N, t + L * r, col, N, 16));
+      v[r].x += static_cast<P>(wv.x);
+      v[r].y += static_cast<P>(wv.y);
+      if constexpr (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+  const double shift = -0.5 * static_cast<double>(N - 1);
+  const int crow = (N * N - 1) / 2 / N, ccol = (N * N - 1) / 2 % N;
+  double sw = 0.0, s3 = 0.0, s4 = 0.0, s5 = 0.0, s6 = 0.0;
+  fftr::static_for<0, R>([&](auto ic) {
+    constexpr int r = decltype(ic)::value;
+    bstore<0>(ru, o1 + r * ostep1, v[r]);
+    const int row = t + L * r;
+    if (partials && col < N && row < N) {
+      const double re = v[r].x, im = v[r].y;
+      const double wei = re * re + im * im;
+      const double dy = row + shift;
+      sw += wei;
+      s3 += dy * wei;
+      s4 += dy * dy * wei;
+      s5 += re;
+      s6 += im;
+      if (row == crow && col == ccol) {
+        partials[static_cast<int64_t>(nslice) * ntile * 8 + 2 * p] = re;
+        partials[static_cast<int64_t>(nslice) * ntile * 8 + 2 * p + 1] = im;
+      }
+    }
+  });
+  if (partials) {
+    const double dx = col + shift;
+    const double acc[7] = {sw, dx * sw, dx * dx * sw, s3, s4, s5, s6};
+#pragma unroll
+    for (int k = 0; k < 7; ++k) {
+      const double a = wave_total(acc[k]);
+      if (lane == 0) red[wave][k] = a;
+    }
+    __syncthreads();
+    if (threadIdx.x < 7) {
+      double a = 0.0;
+      for (int w = 0; w < C::kWaves; ++w) a += red[w][threadIdx.x];
+      partials[(static_cast<int64_t>(p) * ntile + tile) * 8 + threadIdx.x] = a;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Sizes N from 257 to 511 with the propagator: convolution through M-point
 // transforms.  One line's step IDFT_N(P . DFT_N(u)) is the circular
 // convolution of u with h = IDFT_N(P); with g_j = h_((j - N + 1) mod N) for
 // j <= 2N - 2 it is the linear convolution (u * g) at N - 1 ... 2N - 2, and a
@@ -800,14 +1039,17 @@ __global__ __launch_bounds__((ConvCfg<P, M>::kThreads)) void fft_cols_conv_kerne
 
 bool is_pow2(int g) { return g >= 2 && (g & (g - 1)) == 0; }
 
-// Points M of the power-of-two transforms that step a line of G points by
-// convolution (sizes that are not powers of two, up to 512), else 0.
-int conv_points(int G) {
-  if (G < 3 || G > 512 || is_pow2(G)) return 0;
-  int m = 2;
-  while (m < 2 * G - 1) m *= 2;
-  return m;
+// Points Q of the transform pairs that step a line of G points by convolution
+// (sizes below 256 that are not powers of two), else 0.
+int half_points(int G) {
+  if (G < 3 || G > 256 || is_pow2(G)) return 0;
+  int q = 2;
+  while (q < G) q *= 2;
+  return q;
 }
+// Points M of the transforms that step larger lines by convolution (257 to
+// 511), else 0.
+int conv_points(int G) { return G > 256 && G < 512 ? 1024 : 0; }
 
 // Launch shape of the DFT kernels (sizes that are not powers of two).
 struct DftCfg {
@@ -877,6 +1119,48 @@ void cols_conv(Field* f, typename C2<P>::T* data, int add_src, int clear, double
                      f->fft_work.get(), partials);
 }
 
+template <class P, int Q>
+void rows_half(Field* f, typename C2<P>::T* data) {
+  using C = HalfCfg<P, Q>;
+  constexpr int LPW = fftr::Shape<Q>::LPW;
+  const int N = f->ngrid;
+  const int64_t nrows = static_cast<int64_t>(f->nslice) * N;
+  const int64_t ngroups = (nrows + LPW - 1) / LPW;
+  const int64_t nblk = std::min<int64_t>((ngroups + C::kWaves - 1) / C::kWaves, 8192);
+  hipLaunchKernelGGL((fft_rows_half_kernel<P, Q>), dim3(static_cast<unsigned>(nblk)),
+                     dim3(C::kThreads), 0, f->ctx->stream, data, nrows, N, f->fft_tw_conv.get(),
+                     f->fft_prop);
+}
+
+template <class P, int Q>
+void cols_half(Field* f, typename C2<P>::T* data, int add_src, int clear, double* partials) {
+  using T2 = typename C2<P>::T;
+  using C = HalfCfg<P, Q>;
+  const int N = f->ngrid;
+  const int ntile = (N + C::TW - 1) / C::TW;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((f->nslice + 7) / 8 * 8 * ntile), dim3(C::kThreads), 0,
+                       f->ctx->stream, data, f->nslice, N, f->fft_tw_conv.get(), f->fft_prop,
+                       static_cast<T2*>(f->src()), f->src_rect.get(), f->first, add_src, clear,
+                       f->fft_work.get(), partials);
+  };
+  go(add_src == 2 ? fft_cols_half_kernel<P, Q, true> : fft_cols_half_kernel<P, Q, false>);
+}
+
+// Calls fn with the compile-time size Q of the transform pairs.
+template <class Fn>
+void with_half(int Q, Fn&& fn) {
+  switch (Q) {
+    case 4: fn(std::integral_constant<int, 4>{}); break;
+    case 8: fn(std::integral_constant<int, 8>{}); break;
+    case 16: fn(std::integral_constant<int, 16>{}); break;
+    case 32: fn(std::integral_constant<int, 32>{}); break;
+    case 64: fn(std::integral_constant<int, 64>{}); break;
+    case 128: fn(std::integral_constant<int, 128>{}); break;
+    default: fn(std::integral_constant<int, 256>{}); break;
+  }
+}
+
 // Calls fn with the compile-time size G (powers of two 2..1024).
 template <class Fn>
 void with_pow2(int G, Fn&& fn) {
@@ -897,14 +1181,16 @@ void with_pow2(int G, Fn&& fn) {
 
 // Columns per workgroup tile of the column pass.
 int col_tile(int G, size_t esz) {
-  if (const int M = conv_points(G)) {
+  if (const int Q = half_points(G)) {
     int tc = 0;
-    with_pow2(M, [&](auto m) {
-      constexpr int mv = decltype(m)::value;
-      tc = esz == sizeof(double2) ? ConvCfg<double, mv>::TW : ConvCfg<float, mv>::TW;
+    with_half(Q, [&](auto q) {
+      constexpr int qv = decltype(q)::value;
+      tc = esz == sizeof(double2) ? HalfCfg<double, qv>::TW : HalfCfg<float, qv>::TW;
     });
     return tc;
   }
+  if (conv_points(G))
+    return esz == sizeof(double2) ? ConvCfg<double, 1024>::TW : ConvCfg<float, 1024>::TW;
   if (!is_pow2(G)) return dft_cfg(G, esz).tc;
   int tc = 0;
   with_pow2(G, [&](auto g) {
@@ -923,8 +1209,12 @@ void run_rows(Field* f, typename C2<P>::T* data, int mode, double scale) {
       with_pow2(G, [&](auto g) { rows_reg<P, decltype(g)::value>(f, data, mode, scale); });
       return;
     }
-    if (mode == ROW_PROP && conv_points(G)) {  // the table holds the normalisation
-      with_pow2(conv_points(G), [&](auto m) { rows_conv<P, decltype(m)::value>(f, data); });
+    if (mode == ROW_PROP && half_points(G)) {  // the tables hold the normalisation
+      with_half(half_points(G), [&](auto q) { rows_half<P, decltype(q)::value>(f, data); });
+      return;
+    }
+    if (mode == ROW_PROP && conv_points(G)) {
+      rows_conv<P, 1024>(f, data);
       return;
     }
     const DftCfg c = dft_cfg(G, sizeof(T2));
@@ -943,7 +1233,8 @@ void run_cols(Field* f, typename C2<P>::T* data, int mode, double scale, int add
   using T2 = typename C2<P>::T;
   const int G = f->ngrid;
   // the register passes can zero the source cells that they add
-  clear = clear && add_src == 1 && mode == COL_PROP && (is_pow2(G) || conv_points(G));
+  clear = clear && add_src == 1 && mode == COL_PROP &&
+          (is_pow2(G) || half_points(G) || conv_points(G));
   const int clr = clear ? 1 : 0;
   f->ctx->launch(G4H_K_FFT_COLS, [&] {
     if (is_pow2(G)) {
@@ -952,10 +1243,14 @@ void run_cols(Field* f, typename C2<P>::T* data, int mode, double scale, int add
       });
       return;
     }
-    if (mode == COL_PROP && conv_points(G)) {
-      with_pow2(conv_points(G), [&](auto m) {
-        cols_conv<P, decltype(m)::value>(f, data, add_src, clr, partials);
+    if (mode == COL_PROP && half_points(G)) {
+      with_half(half_points(G), [&](auto q) {
+        cols_half<P, decltype(q)::value>(f, data, add_src, clr, partials);
       });
+      return;
+    }
+    if (mode == COL_PROP && conv_points(G)) {
+      cols_conv<P, 1024>(f, data, add_src, clr, partials);
       return;
     }
     const DftCfg c = dft_cfg(G, sizeof(T2));
@@ -998,12 +1293,12 @@ void fft_step(Field* f, bool source_on, bool stats, bool clear) {
   run_cols<P>(f, data, COL_PROP, invg, add, partials, clear);
 }
 
-// The M-point convolution table of a line step with factors P (natural
-// frequency order, N points): h = IDFT_N(P), g_j = h_((j - N + 1) mod N) for
-// j <= 2N - 2 (zero beyond), H = DFT_M(g) / M, stored in the pi order of the
-// M-point register transforms.  Sums in long double over exact twiddle
-// indices, so the table is correctly rounded to a few ulp.
-std::vector<double2> conv_spectrum(const std::vector<double2>& P, int M) {
+// The M-point convolution spectrum of a line step with factors P (natural
+// frequency order, N points): h = IDFT_N(P), g_j = h_((j - shift) mod N) at
+// j mod M for shift - N < j < shift + N, H = DFT_M(g) / M.  Sums in long
+// double over exact twiddle indices, so the table is correctly rounded to a
+// few ulp.
+std::vector<double2> conv_spectrum(const std::vector<double2>& P, int M, int shift) {
   using LD = long double;
   const int N = static_cast<int>(P.size());
   const LD pi2 = 8 * std::atan(static_cast<LD>(1));
@@ -1030,16 +1325,34 @@ std::vector<double2> conv_spectrum(const std::vector<double2>& P, int M) {
   std::vector<double2> out(M);
   for (int k = 0; k < M; ++k) {  // H_k = (1/M) sum_j g_j e^{-2 pi i j k / M}
     LD ar = 0, ai = 0;
-    for (int j = 0; j <= 2 * N - 2; ++j) {
-      const int n = (j - N + 1 + N) % N;
+    for (int d = 1 - N; d < N; ++d) {
+      const int n = (d + N) % N, j = (d + shift + M) % M;
       const int q = static_cast<int>((static_cast<int64_t>(j) * k) % M);
       ar += hr[n] * cm[q] + hi[n] * sm[q];
       ai += hi[n] * cm[q] - hr[n] * sm[q];
     }
     out[k] = make_double2(static_cast<double>(ar / M), static_cast<double>(ai / M));
   }
+  return out;
+}
+
+// The multipliers of the lines' transforms in their pi orders: of M-point
+// lines (results at N - 1 ... 2N - 2), or the even and then the odd ones of
+// the transform pairs (results at 0 ... N - 1).
+std::vector<double2> conv_table(const std::vector<double2>& P, int M) {
+  const int N = static_cast<int>(P.size());
+  const std::vector<double2> out = conv_spectrum(P, M, N - 1);
   std::vector<double2> perm(M);
   for (int e = 0; e < M; ++e) perm[e] = out[fftr::spectrum_index(e, M)];
+  return perm;
+}
+std::vector<double2> half_table(const std::vector<double2>& P, int Q) {
+  const std::vector<double2> out = conv_spectrum(P, 2 * Q, 0);
+  std::vector<double2> perm(2 * Q);
+  for (int e = 0; e < Q; ++e) {
+    perm[e] = out[2 * fftr::spectrum_index(e, Q)];
+    perm[Q + e] = out[2 * fftr::spectrum_index(e, Q) + 1];
+  }
   return perm;
 }
 
@@ -1063,17 +1376,23 @@ void fft_prepare(Field* f, double delz) {
     }
     f->fft_tw.alloc(f->ctx, G);
     G4_HIP(hipMemcpy(f->fft_tw.get(), tw.data(), sizeof(double2) * G, hipMemcpyHostToDevice));
-    if (const int M = conv_points(G)) {
-      // the M-point convolution transforms' four-step twiddles
+    const int Q = half_points(G);
+    if (const int M = Q ? Q : conv_points(G)) {
+      // the convolution transforms' four-step twiddles, and after those of
+      // transform pairs w_n = exp(-2 pi i n / 2Q)
       const int L = fftr::lanes_per_line(M);
-      std::vector<double2> twm(M);
+      std::vector<double2> twm(Q ? 2 * M : M);
       for (int k = 0; k < M; ++k) {
         const int64_t e = static_cast<int64_t>(k % L) * (k / L);
         const double a = -pi2 * static_cast<double>(e % M) / static_cast<double>(M);
         twm[k] = make_double2(std::cos(a), std::sin(a));
       }
-      f->fft_tw_conv.alloc(f->ctx, M);
-      G4_HIP(hipMemcpy(f->fft_tw_conv.get(), twm.data(), sizeof(double2) * M,
+      for (int n = 0; n < Q; ++n) {
+        const double a = -pi2 * static_cast<double>(n) / static_cast<double>(2 * Q);
+        twm[Q + n] = make_double2(std::cos(a), std::sin(a));
+      }
+      f->fft_tw_conv.alloc(f->ctx, twm.size());
+      G4_HIP(hipMemcpy(f->fft_tw_conv.get(), twm.data(), sizeof(double2) * twm.size(),
                        hipMemcpyHostToDevice));
     }
     f->fft_delz = 0.0;
@@ -1118,7 +1437,10 @@ void fft_prepare(Field* f, double delz) {
         const double ph = -dx * dx * dk * dk / 2. / f->xks * delz;
         t.host[e] = make_double2(std::cos(ph), std::sin(ph));
       }
-      if (const int M = conv_points(G)) t.host = conv_spectrum(t.host, M);
+      if (const int Q = half_points(G))
+        t.host = half_table(t.host, Q);
+      else if (const int M = conv_points(G))
+        t.host = conv_table(t.host, M);
       t.dev.alloc(f->ctx, t.host.size());
       G4_HIP(hipMemcpyAsync(t.dev.get(), t.host.data(), sizeof(double2) * t.host.size(),
                             hipMemcpyHostToDevice, f->ctx->stream));
