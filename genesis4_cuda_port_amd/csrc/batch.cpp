@@ -34,6 +34,7 @@
 // Steady state only: one slice per run, no slippage (Gencore.cpp:229 is a
 // no-op there, ControlCUDA.cpp:150).
 #include <algorithm>
+#include <cstring>
 #include <map>
 #include <memory>
 #include <tuple>
@@ -146,6 +147,22 @@ struct g4h_batch {
     nrec = 1;
   }
 
+  // Whether two steps differ at most in position and what they record.
+  static bool same_physics(g4h_step a, g4h_step b) {
+    a.z = b.z = 0.0;
+    a.outstep = b.outstep = a.marker = b.marker = 0;
+    return std::memcmp(&a, &b, sizeof(g4h_step)) == 0;
+  }
+  // Beam sums of a step's parameters to record rk (none if rk < 0).
+  void set_record(ParticleParams& p, const Group& g, int rk) const {
+    p.stages &= ~ST_DIAG;
+    p.diag = DiagParams{};
+    if (rk < 0) return;
+    p.stages |= ST_DIAG;
+    p.diag.raw = g.beam_hist.get() + static_cast<size_t>(rk) * beam_rec(g);
+    p.diag.nharm = nharm;
+  }
+
   // Every step's parameter table of every group, built on the host with the
   // same make_trans / make_push / make_dep as every other path and uploaded
   // once, so that a step enqueues launches only.
@@ -169,6 +186,16 @@ struct g4h_batch {
           g4h_step st = st0;
           const auto& a = aw[static_cast<size_t>(g.runs[static_cast<size_t>(i)])];
           if (!a.empty()) st.aw = a[static_cast<size_t>(k)];
+          const int rk = rec[static_cast<size_t>(k)];
+          if (k > 0 && same_physics(st0, steps[static_cast<size_t>(k - 1)]) &&
+              (a.empty() || a[static_cast<size_t>(k)] == a[static_cast<size_t>(k - 1)])) {
+            // as the step before, records apart (a module is many such steps)
+            ParticleParams& q = tab[static_cast<size_t>(k) * n + i];
+            q = tab[static_cast<size_t>(k - 1) * n + i];
+            set_record(q, g, rk);
+            src_on = g.src_on[static_cast<size_t>(k - 1)] != 0;
+            continue;
+          }
           ParticleParams p{};
           p.gamma0 = g.gamma0;
           p.stages = ST_T1 | ST_PUSH | ST_T2;
@@ -182,12 +209,7 @@ struct g4h_batch {
           require(i == 0 || on == src_on, "source switched on for part of a batch group");
           src_on = on;
           if (on) p.stages |= ST_DEP;
-          const int rk = rec[static_cast<size_t>(k)];
-          if (rk >= 0) {
-            p.stages |= ST_DIAG;
-            p.diag.raw = g.beam_hist.get() + static_cast<size_t>(rk) * beam_rec(g);
-            p.diag.nharm = nharm;
-          }
+          set_record(p, g, rk);
           tab[static_cast<size_t>(k) * n + i] = p;
         }
         g.head[static_cast<size_t>(k)] = tab[static_cast<size_t>(k) * n];
@@ -524,9 +546,18 @@ g4h_status g4h_batch_create(g4h_context* ctx, g4h_precision precision, g4h_solve
       off[static_cast<size_t>(i) + 1] = off[static_cast<size_t>(i)] + q.npart;
       cur[static_cast<size_t>(i)] = q.current;
     }
-    const size_t np = static_cast<size_t>(off.back());
-    std::vector<double> x(np), y(np), px(np), py(np), ga(np), th(np);
-    std::vector<double> re(static_cast<size_t>(n) * g.G * g.G), im(re.size());
+    ok(g4h_context_create(ctx->device, &g.gctx));
+    ok(g4h_beam_create(g.gctx, precision, n, off.data(), cur.data(), g.gamma0, &g.beam));
+    ok(g4h_field_create(g.gctx, precision, n, g.G, g.gridmax, lambda0, lambda0, 1, &g.field));
+    // initial state on the device, as g4h_beam_generate makes it, and one
+    // seed plane per distinct seed of the group; on the host the loader and
+    // 3 M exponentials of the planes took most of a 96-run batch's creation
+    DevBuf<double> dcur, dseed;
+    dcur.alloc(g.gctx, static_cast<size_t>(n));
+    G4_HIP(hipMemcpy(dcur.get(), cur.data(), sizeof(double) * cur.size(), hipMemcpyHostToDevice));
+    const size_t plane = static_cast<size_t>(g.G) * g.G;
+    std::vector<double> re, im;
+    std::pair<double, double> have(0.0, 0.0);  // power, w0 of the plane in dseed
     for (int i = 0; i < n; ++i) {
       const g4h_batch_run& q = runs[g.runs[static_cast<size_t>(i)]];
       g4h_beam_spec s{};
@@ -544,20 +575,22 @@ g4h_status g4h_batch_create(g4h_context* ctx, g4h_precision precision, g4h_solve
       s.nbins = q.nbins;
       s.shotnoise = q.shotnoise;
       s.seed = q.seed;
-      const size_t o = static_cast<size_t>(off[static_cast<size_t>(i)]);
-      ok(g4h_load_beam(&s, &q.current, x.data() + o, y.data() + o, px.data() + o, py.data() + o,
-                       ga.data() + o, th.data() + o));
+      launch_generate_slice(g.beam, i, &s, dcur.get() + i);
       if (q.seed_power > 0) {
-        const size_t po = static_cast<size_t>(i) * g.G * g.G;
-        ok(g4h_seed_gaussian(1, g.G, g.gridmax, lambda0, q.seed_power, q.seed_w0, re.data() + po,
-                             im.data() + po));
+        if (re.empty() || have != std::make_pair(q.seed_power, q.seed_w0)) {
+          re.resize(plane);
+          im.resize(plane);
+          ok(g4h_seed_gaussian(1, g.G, g.gridmax, lambda0, q.seed_power, q.seed_w0, re.data(),
+                               im.data()));
+          G4_HIP(hipStreamSynchronize(g.gctx->stream));  // the plane before may be in use
+          if (dseed.empty()) dseed.alloc(g.gctx, plane);
+          G4_HIP(hipMemcpy(dseed.get(), re.data(), sizeof(double) * plane, hipMemcpyHostToDevice));
+          have = {q.seed_power, q.seed_w0};
+        }
+        launch_set_plane(g.field, i, dseed.get());
       }
     }
-    ok(g4h_context_create(ctx->device, &g.gctx));
-    ok(g4h_beam_create(g.gctx, precision, n, off.data(), cur.data(), g.gamma0, &g.beam));
-    ok(g4h_beam_upload(g.beam, x.data(), y.data(), px.data(), py.data(), ga.data(), th.data()));
-    ok(g4h_field_create(g.gctx, precision, n, g.G, g.gridmax, lambda0, lambda0, 1, &g.field));
-    ok(g4h_field_upload(g.field, re.data(), im.data(), 0));
+    g.field->uploaded = true;
     ok(g4h_field_init_solver(g.field, solver, 0, 1.0, 1.0, 1.0, 0));
     G4_HIP(hipEventCreateWithFlags(&g.tail, hipEventDisableTiming));
     g.beam_hist.alloc(g.gctx, static_cast<size_t>(b->cap) * b->beam_rec(g));
@@ -625,18 +658,28 @@ g4h_status g4h_batch_download(g4h_batch* b, int run, double* beam_raw, double* f
   const auto [gi, si] = b->where[static_cast<size_t>(run)];
   const Group& g = b->groups[static_cast<size_t>(gi)];
   G4_HIP(hipStreamSynchronize(g.gctx->stream));
-  const size_t br = G4H_BEAM_RAW(b->nharm);
-  for (int r = 0; r < b->nrec; ++r) {
-    if (beam_raw)
-      G4_HIP(hipMemcpy(beam_raw + static_cast<size_t>(r) * br,
-                       g.beam_hist.get() + static_cast<size_t>(r) * b->beam_rec(g) + si * br,
-                       sizeof(double) * br, hipMemcpyDeviceToHost));
-    if (field_raw)
-      G4_HIP(hipMemcpy(field_raw + static_cast<size_t>(r) * G4H_FIELD_RAW,
-                       g.field_hist.get() + static_cast<size_t>(r) * b->field_rec(g) +
-                           static_cast<size_t>(si) * G4H_FIELD_RAW,
-                       sizeof(double) * G4H_FIELD_RAW, hipMemcpyDeviceToHost));
-  }
+  // the run's rows of the group's records, gathered on the device so that
+  // one copy brings them over (a copy per record was 20 us each)
+  const size_t br = G4H_BEAM_RAW(b->nharm), fr = G4H_FIELD_RAW;
+  const size_t n = static_cast<size_t>(b->nrec);
+  if (n == 0) return G4H_OK;
+  DevBuf<double> rows;
+  rows.alloc(g.gctx, n * (br + fr));
+  auto gather = [&](double* to, const double* from, size_t width, size_t pitch) {
+    G4_HIP(hipMemcpy2DAsync(to, sizeof(double) * width, from, sizeof(double) * pitch,
+                            sizeof(double) * width, n, hipMemcpyDeviceToDevice, g.gctx->stream));
+  };
+  if (beam_raw)
+    gather(rows.get(), g.beam_hist.get() + static_cast<size_t>(si) * br, br, b->beam_rec(g));
+  if (field_raw)
+    gather(rows.get() + n * br, g.field_hist.get() + static_cast<size_t>(si) * fr, fr,
+           b->field_rec(g));
+  G4_HIP(hipStreamSynchronize(g.gctx->stream));
+  if (beam_raw)
+    G4_HIP(hipMemcpy(beam_raw, rows.get(), sizeof(double) * n * br, hipMemcpyDeviceToHost));
+  if (field_raw)
+    G4_HIP(hipMemcpy(field_raw, rows.get() + n * br, sizeof(double) * n * fr,
+                     hipMemcpyDeviceToHost));
   G4_API_END
 }
 

@@ -298,6 +298,10 @@ void make_push(PushParams& p, const g4h_step& st, double gamma0, double delz,
                Field* const* fields, int nfield, const double* d_eloss);
 bool make_dep(DepParams& d, Field* f, Beam* b, const g4h_step& st, double delz);
 
+// ---- initial state -------------------------------------------------------
+void launch_generate_slice(Beam* b, int slice, const g4h_beam_spec* spec, const double* d_current);
+void launch_set_plane(Field* f, int slot, const double* d_re);
+
 // ---- field solvers -------------------------------------------------------
 void field_prepare_solver(Field* f, double delz);  // (re)build coefficient tables
 void* field_adi_ustar(Field* f);  // the ADI x sweep's output planes (allocated on first use)

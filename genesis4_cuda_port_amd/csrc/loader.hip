@@ -39,6 +39,17 @@ __global__ void beam_generate_kernel(loader::Spec sp, const double* current, dou
   }
 }
 
+// one ring plane <- a real plane
+template <class T2>
+__global__ void set_plane_kernel(const double* re, int64_t plane, T2* u) {
+  const int64_t e = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (e >= plane) return;
+  T2 v;
+  v.x = re[e];
+  v.y = 0;
+  u[e] = v;
+}
+
 // every ring plane <- the plane `src`
 template <class T2>
 __global__ void fill_planes_kernel(const T2* src, int64_t plane, int nslice, T2* u) {
@@ -49,6 +60,46 @@ __global__ void fill_planes_kernel(const T2* src, int64_t plane, int nslice, T2*
 }
 
 }  // namespace
+
+// Slice `slice` of the beam from a one-slice specification; d_current: the
+// slice current on the device (shot noise).  Enqueued on the beam's stream.
+void launch_generate_slice(Beam* b, int slice, const g4h_beam_spec* spec,
+                           const double* d_current) {
+  loader::Spec sp;
+  require(loader_spec(spec, sp) && spec->nslice == 1, "invalid beam specification");
+  const int64_t o = b->off_h[static_cast<size_t>(slice)];
+  require(b->off_h[static_cast<size_t>(slice) + 1] - o == spec->npart,
+          "beam slice and specification differ in particle count");
+  const unsigned blocks = static_cast<unsigned>((spec->npart / spec->nbins + 255) / 256);
+  b->ctx->launch(G4H_K_OTHER, [&] {
+    if (b->prec == G4H_FP64)
+      hipLaunchKernelGGL(beam_generate_kernel<double>, dim3(blocks), dim3(256), 0, b->ctx->stream,
+                         sp, d_current, b->gamma_ref, b->xd.get() + o, b->yd.get() + o,
+                         b->pxd.get() + o, b->pyd.get() + o, b->gd.get() + o, b->theta.get() + o);
+    else
+      hipLaunchKernelGGL(beam_generate_kernel<float>, dim3(blocks), dim3(256), 0, b->ctx->stream,
+                         sp, d_current, b->gamma_ref, b->xf.get() + o, b->yf.get() + o,
+                         b->pxf.get() + o, b->pyf.get() + o, b->gf.get() + o, b->theta.get() + o);
+  });
+  b->uploaded = true;
+  b->touched();
+}
+
+// Ring plane `slot` of the field from a real plane of ngrid^2 values on the
+// device; enqueued on the field's stream.
+void launch_set_plane(Field* f, int slot, const double* d_re) {
+  const int64_t plane = static_cast<int64_t>(f->ngrid) * f->ngrid;
+  const unsigned blocks = static_cast<unsigned>((plane + 255) / 256);
+  f->ctx->launch(G4H_K_OTHER, [&] {
+    if (f->prec == G4H_FP64)
+      hipLaunchKernelGGL(set_plane_kernel<double2>, dim3(blocks), dim3(256), 0, f->ctx->stream,
+                         d_re, plane, f->ud.get() + slot * plane);
+    else
+      hipLaunchKernelGGL(set_plane_kernel<float2>, dim3(blocks), dim3(256), 0, f->ctx->stream,
+                         d_re, plane, f->uf.get() + slot * plane);
+  });
+}
+
 }  // namespace g4
 
 using namespace g4;
