@@ -377,9 +377,7 @@ struct g4h_batch {
       if (f->adi_y.size() < static_cast<size_t>(f->cells())) f->adi_y.alloc(f->ctx, f->cells());
       ensure_source(f);
       (void)field_adi_ustar(f);
-      const int nblk = (g.G + kAdiSegLines - 1) / kAdiSegLines;
-      const size_t need = g.runs.size() * static_cast<size_t>(nblk) * 8 + 2 * g.runs.size();
-      if (f->col_partials.size() < need) f->col_partials.alloc(f->ctx, need);
+      field_stats_reserve(f);
       dadi[gi].alloc(g.gctx, static_cast<size_t>(ns));
       dcs[gi].alloc(g.gctx, static_cast<size_t>(ns));
       G4_HIP(hipMemcpyAsync(dadi[gi].get(), fac.data(), sizeof(const double2*) * ns,

@@ -623,8 +623,7 @@ void adi_step(Field* f, bool source_on, bool stats, bool clear) {
     return;
   }
   if (stats) {
-    if (f->plane_stats.size() != static_cast<size_t>(f->nslice) * G4H_FIELD_RAW)
-      f->plane_stats.alloc(f->ctx, static_cast<size_t>(f->nslice) * G4H_FIELD_RAW);
+    field_stats_reserve(f);
     f->stats_ntile = 0;
   }
   f->ctx->launch(G4H_K_ADI_X, [&] {

@@ -1271,7 +1271,7 @@ void fft_step(Field* f, bool source_on, bool stats, bool clear) {
   const int G = f->ngrid;
   T2* data = static_cast<T2*>(f->data());
   const double invg = 1.0 / static_cast<double>(G);
-  const int ntile = (G + col_tile(G, sizeof(T2)) - 1) / col_tile(G, sizeof(T2));
+  const int ntile = fft_stat_tiles(f);
   double* partials = nullptr;
   if (stats) partials = field_partials(f, ntile);
   int add = source_on ? 1 : 0;
@@ -1458,6 +1458,9 @@ void fft_solve(Field* f, bool source_on, bool stats, bool clear) {
     fft_step<float>(f, source_on, stats, clear);
 }
 
-bool fft_supported(int G) { return G >= 2 && G <= 1024; }
+int fft_stat_tiles(const Field* f) {
+  const int tc = col_tile(f->ngrid, f->prec == G4H_FP64 ? sizeof(double2) : sizeof(float2));
+  return (f->ngrid + tc - 1) / tc;
+}
 
 }  // namespace g4

@@ -10,6 +10,8 @@ void fft_solve(Field* f, bool source_on, bool stats, bool clear);
 
 namespace {
 
+constexpr int kStatTiles = 16;  // most tiles per plane of any ADI or standalone sums
+
 // The end of a step: zero fill of the planes that slippage brought in
 // (ControlCUDA.cpp:237-244) and, with raw, the field record of every slice
 // from the solver's per-tile sums, in one launch.  In logical slice order
@@ -126,9 +128,19 @@ __global__ void reset_rect_kernel(int4* rect, int4* bbox, int n) {
 
 }  // namespace
 
-double* field_partials(Field* f, int ntile) {
-  const size_t need = static_cast<size_t>(f->nslice) * (static_cast<size_t>(ntile) * 8 + 2);
+// ceil(1024 / 64) line blocks of the lane sweeps, ceil(256 / 16) of the
+// segmented ones and plane_stats_kernel's limit all come to 16.
+void field_stats_reserve(Field* f) {
+  const int ntile = f->kind == G4H_SOLVER_FFT ? std::max(kStatTiles, fft_stat_tiles(f)) : kStatTiles;
+  const size_t n = static_cast<size_t>(f->nslice);
+  const size_t need = n * (static_cast<size_t>(ntile) * 8 + 2);
   if (f->col_partials.size() < need) f->col_partials.alloc(f->ctx, need);
+  if (f->kind == G4H_SOLVER_ADI && f->plane_stats.empty())
+    f->plane_stats.alloc(f->ctx, n * G4H_FIELD_RAW);
+}
+
+double* field_partials(Field* f, int ntile) {
+  field_stats_reserve(f);
   f->stats_ntile = ntile;
   return f->col_partials.get();
 }
@@ -201,7 +213,7 @@ void field_solve(Field* f, bool source_on, bool stats, bool clear) {
 void field_plane_stats(Field* f) {
   // enough workgroups to fill the GPU from few planes, at least 4 rows each
   const int ntile =
-      std::max(1, std::min({16, (1024 + f->nslice - 1) / f->nslice, (f->ngrid + 3) / 4}));
+      std::max(1, std::min({kStatTiles, (1024 + f->nslice - 1) / f->nslice, (f->ngrid + 3) / 4}));
   double* partials = field_partials(f, ntile);
   const dim3 grid(static_cast<unsigned>(f->nslice) * ntile);
   f->ctx->launch(G4H_K_OTHER, [&] {

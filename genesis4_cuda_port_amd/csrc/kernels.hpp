@@ -312,6 +312,12 @@ void* field_adi_ustar(Field* f);  // the ADI x sweep's output planes (allocated 
 // reads them, where that pass can (f->src_clear tells).
 void field_solve(Field* f, bool source_on, bool stats, bool clear = false);
 void field_plane_stats(Field* f);                      // standalone field sums
+// Room for the field sums of every pass that may run on the field with its
+// present solver, whichever variant and tile count: taken at once, so that
+// the buffers a captured run writes to are neither replaced by a later eager
+// pass nor first needed inside a capture.
+void field_stats_reserve(Field* f);
+int fft_stat_tiles(const Field* f);  // tiles per plane of the FFT column pass
 // Room for per-tile field sums partials[(p*ntile + t)*8 + k] (k < 7) and the
 // centre cells at partials[nslice*ntile*8 + 2p]; makes them the planes' sums.
 double* field_partials(Field* f, int ntile);

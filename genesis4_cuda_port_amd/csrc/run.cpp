@@ -282,6 +282,7 @@ g4h_status g4h_run_capture(g4h_run* r) {
     if (r->f->delz_tables.size() + missing > Field::kMaxDelzTables) r->f->evict_delz_tables();
     for (double d : lens) field_prepare_solver(r->f, d);
   }
+  field_stats_reserve(r->f);
   G4_HIP(hipStreamSynchronize(ctx->stream));
   ctx->tune_settle();
   if (r->b->prec == G4H_FP64) {

@@ -19,7 +19,7 @@ from _oracle import OField
 import cases
 from cases import GAMMA0, LAMBDA0, quad_step
 from genesis4_cuda_port_amd import api
-from genesis4_cuda_port_amd._abi import G4Error
+from genesis4_cuda_port_amd._abi import TUNE_ADI, G4Error
 
 pytestmark = pytest.mark.gpu
 
@@ -124,6 +124,71 @@ def test_replay_refused_after_table_eviction(kind):
         # the stream is out of capture mode: eager work still runs
         b.diag_raw(1)
         ctx.synchronize()
+        run.close()
+        f.close()
+        b.close()
+
+
+def _replayed(ctx, run, f, c):
+    f.upload(c.seed_re, c.seed_im, 0)
+    run.replay()
+    return run.download_diag()[1]
+
+
+def test_replay_keeps_its_sums_buffers():
+    """A run captured with one ADI variant, replayed after an eager run through
+    variants whose field sums have more tiles per plane (9 line blocks of 16
+    against the standalone sums' 4 tiles, and the workgroup variant's whole
+    sums) and after other allocations: every replay gives the field records of
+    the eager run.  No current, so the records are equal bit for bit."""
+    print("case replay_sums_buffers", flush=True)
+    c = cases.make_case(nslice=300, npart=64, ngrid=129, nsteps=3, seed_power=1e4, current=0.0)
+    with api.Context(0) as ctx:
+        ctx.set_variant(TUNE_ADI, 0)
+        b = gpu_beam(ctx, c, api.MIXED)
+        f = gpu_field(ctx, c, api.MIXED)
+        run = api.Run(ctx, b, f, c.steps, LAMBDA0, c.sample, c.timerun, False, 1)
+        run.advance(len(c.steps))
+        ref = run.download_diag()[1]
+        run.capture()
+        held = []
+        for rep in range(3):
+            assert np.array_equal(_replayed(ctx, run, f, c), ref)
+            ctx.set_variant(TUNE_ADI, (-1, 1, 2)[rep])
+            f.upload(c.seed_re, c.seed_im, 0)
+            other = api.Run(ctx, b, f, c.steps, LAMBDA0, c.sample, c.timerun, False, 1)
+            other.advance(len(c.steps))
+            held.append(other)
+            for n in (8, 64):  # buffers that would take over released memory
+                g = api.Field(ctx, api.FP64, n, 33, c.gridmax, LAMBDA0, c.slicelength)
+                g.diag_raw()
+                held.append(g)
+        assert np.array_equal(_replayed(ctx, run, f, c), ref)
+        for x in held:
+            x.close()
+        run.close()
+        f.close()
+        b.close()
+
+
+def test_capture_before_the_tuner_decides():
+    """Two steps on a grid whose ADI variant is still being tried: the only
+    record falls on the second trial, and the capture takes variant 0, whose
+    sums the eager pass never needed.  The capture must not have to allocate
+    them, and the replay equals the eager records (the variants are
+    bit-identical)."""
+    print("case capture_undecided", flush=True)
+    c = cases.make_case(nslice=2, npart=64, ngrid=283, nsteps=2, seed_power=1e4, current=0.0)
+    c.steps[0].outstep = 0
+    with api.Context(0) as ctx:
+        b = gpu_beam(ctx, c, api.FP64)
+        f = gpu_field(ctx, c, api.FP64)
+        run = api.Run(ctx, b, f, c.steps, LAMBDA0, c.sample, c.timerun, False, 1)
+        run.advance(len(c.steps))
+        ref = run.download_diag()[1]
+        assert ref.shape[0] == 2
+        run.capture()
+        assert np.array_equal(_replayed(ctx, run, f, c), ref)
         run.close()
         f.close()
         b.close()
