@@ -960,6 +960,29 @@ struct SplitScratch {
   int atomic_win;
 };
 
+// Folds the cells that particles [i0, i1) touch into LDS box[0..3] (min x,
+// min y, max x, max y; set empty before); valid after the next barrier.
+template <class P>
+__device__ __forceinline__ void fold_footprint(BeamPtr<P> b, int64_t i0, int64_t i1,
+                                               const DepParams& d, int* box) {
+  int mnx = 0x7fffffff, mny = 0x7fffffff, mxx = -1, mxy = -1;
+  for (int64_t k = i0 + threadIdx.x; k < i1; k += blockDim.x) {
+    int ix, iy;
+    P wx, wy;
+    if (cell_of<P>(b.x[k], b.y[k], P(d.gridmax), P(d.dgrid), P(d.inv_dgrid), d.ngrid, ix, iy, wx,
+                   wy)) {
+      mnx = min(mnx, ix);
+      mny = min(mny, iy);
+      mxx = max(mxx, ix + 1);
+      mxy = max(mxy, iy + 1);
+    }
+  }
+  atomicMin(&box[0], mnx);
+  atomicMin(&box[1], mny);
+  atomicMax(&box[2], mxx);
+  atomicMax(&box[3], mxy);
+}
+
 // The deposition window of a slice: the cells it touched last step (bb)
 // plus a 2-cell margin, clipped to the grid and to cap cells (centred);
 // empty without a footprint or without current.
@@ -1263,22 +1286,7 @@ __device__ __forceinline__ void particle_slice(BeamPtr<P> b, const int32_t* off,
         s_bb[2] = s_bb[3] = -1;
       }
       __syncthreads();
-      int mnx = 0x7fffffff, mny = 0x7fffffff, mxx = -1, mxy = -1;
-      for (int64_t k = i0s + tid; k < i1s; k += NT) {
-        int ix, iy;
-        P wx, wy;
-        if (cell_of<P>(b.x[k], b.y[k], P(prm.dep.gridmax), P(prm.dep.dgrid),
-                       P(prm.dep.inv_dgrid), ng, ix, iy, wx, wy)) {
-          mnx = min(mnx, ix);
-          mny = min(mny, iy);
-          mxx = max(mxx, ix + 1);
-          mxy = max(mxy, iy + 1);
-        }
-      }
-      atomicMin(&s_bb[0], mnx);
-      atomicMin(&s_bb[1], mny);
-      atomicMax(&s_bb[2], mxx);
-      atomicMax(&s_bb[3], mxy);
+      fold_footprint(b, i0s, i1s, prm.dep, s_bb);
       __syncthreads();
       bb = make_int4(s_bb[0], s_bb[1], s_bb[2], s_bb[3]);
       __syncthreads();
@@ -1535,12 +1543,14 @@ __global__ __launch_bounds__(kThreads) void particle_kernel(BeamPtr<P> b, const 
 // the other, took 17.7 us at one slice and K = 4.
 template <class P, bool TAB>
 __global__ __launch_bounds__(kThreads) void split_combine_kernel(
-    const int32_t* off, ParticleParams prm_arg, const ParticleParams* __restrict__ tab,
+    BeamPtr<P> b, const int32_t* off, ParticleParams prm_arg, const ParticleParams* __restrict__ tab,
     SplitScratch sp, int K) {
   using T2 = typename V2<P>::T;
   const ParticleParams& prm = slice_params<TAB, P>(prm_arg, tab);
   const int s = blockIdx.x;
   const int tid = threadIdx.x;
+  __shared__ int s_bb[4];
+  __shared__ int s_none;
   if (blockIdx.y + 1 < gridDim.y) {
     const int4 wb = sp.wb[s];
     const int k = blockIdx.y * kThreads + tid;
@@ -1580,6 +1590,22 @@ __global__ __launch_bounds__(kThreads) void split_combine_kernel(
       const int4 wb = sp.wb[s];
       const int bb[4] = {t.x, t.y, t.z, t.w}, fb[4] = {f.x, f.y, f.z, f.w};
       publish_boxes(prm, s, wb.x, wb.y, wb.z, wb.w, bb, fb);
+      s_none = t.x > t.z && f.x > f.z;
+      s_bb[0] = s_bb[1] = 0x7fffffff;
+      s_bb[2] = s_bb[3] = -1;
+    }
+  }
+  if (prm.stages & ST_DEP) {
+    // Nothing deposited although the slice has current (a step of zero
+    // strength, or no particle on the grid): without a footprint the next
+    // pass, which may come without a pre-pass, would send every particle
+    // through the global atomics.  The positions after this pass give it.
+    __syncthreads();
+    if (s_none && prm.dep.cur_over_npar[s] != 0.0) {
+      fold_footprint(b, off[s], off[s + 1], prm.dep, s_bb);
+      __syncthreads();
+      if (tid == 0 && s_bb[0] <= s_bb[2])
+        prm.dep.bbox[s] = make_int4(s_bb[0], s_bb[1], s_bb[2], s_bb[3]);
     }
   }
   if (!(prm.stages & ST_DIAG)) return;
@@ -1663,22 +1689,7 @@ __global__ void split_prepass_kernel(BeamPtr<P> b, const int32_t* off, ParticleP
     s_bb[2] = s_bb[3] = -1;
   }
   __syncthreads();
-  int mnx = 0x7fffffff, mny = 0x7fffffff, mxx = -1, mxy = -1;
-  for (int64_t k = off[s] + tid; k < off[s + 1]; k += blockDim.x) {
-    int ix, iy;
-    P wx, wy;
-    if (cell_of<P>(b.x[k], b.y[k], P(prm.dep.gridmax), P(prm.dep.dgrid), P(prm.dep.inv_dgrid), ng,
-                   ix, iy, wx, wy)) {
-      mnx = min(mnx, ix);
-      mny = min(mny, iy);
-      mxx = max(mxx, ix + 1);
-      mxy = max(mxy, iy + 1);
-    }
-  }
-  atomicMin(&s_bb[0], mnx);
-  atomicMin(&s_bb[1], mny);
-  atomicMax(&s_bb[2], mxx);
-  atomicMax(&s_bb[3], mxy);
+  fold_footprint(b, off[s], off[s + 1], prm.dep, s_bb);
   __syncthreads();
   // stays empty when no particle is on the grid: every part then deposits
   // through the global fallback
@@ -1759,7 +1770,7 @@ void launch_t(Context* ctx, Beam* b, const ParticleParams& p, BeamPtr<P> bp,
     const int nwg = DEP ? (p.dep.window_cap + kThreads - 1) / kThreads : 0;
     ctx->launch(G4H_K_OTHER, [&] {
       hipLaunchKernelGGL((split_combine_kernel<P, TAB>), dim3(b->nslice, nwg + 1), dim3(kThreads),
-                         0, ctx->stream, b->off.get(), p, tab, sp, K);
+                         0, ctx->stream, bp, b->off.get(), p, tab, sp, K);
     });
   }
   ctx->param_commit(slot);
@@ -1970,7 +1981,7 @@ void launch_diag_given(Context* ctx, Beam* b, const ParticleParams& p, BeamPtr<P
   if (K > 1) {
     ctx->launch(G4H_K_OTHER, [&] {
       hipLaunchKernelGGL((split_combine_kernel<P, false>), dim3(b->nslice), dim3(kThreads), 0,
-                         ctx->stream, b->off.get(), p, d_prm, sp, K);
+                         ctx->stream, bp, b->off.get(), p, d_prm, sp, K);
     });
   }
 }
