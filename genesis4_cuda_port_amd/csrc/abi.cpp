@@ -628,11 +628,14 @@ g4h_status g4h_field_create(g4h_context* ctx, g4h_precision precision, int nslic
     const size_t cells = static_cast<size_t>(f->cells());
     if (precision == G4H_FP64) {
       f->ud.alloc(ctx, cells);
-      G4_HIP(hipMemset(f->ud.get(), 0, cells * sizeof(double2)));
+      G4_HIP(hipMemsetAsync(f->ud.get(), 0, cells * sizeof(double2), ctx->stream));
     } else {
       f->uf.alloc(ctx, cells);
-      G4_HIP(hipMemset(f->uf.get(), 0, cells * sizeof(float2)));
+      G4_HIP(hipMemsetAsync(f->uf.get(), 0, cells * sizeof(float2), ctx->stream));
     }
+    // cleared before anyone writes planes, on this stream, another one (another
+    // context's work) or by a blocking copy
+    G4_HIP(hipStreamSynchronize(ctx->stream));
   } catch (...) {
     delete f;
     throw;

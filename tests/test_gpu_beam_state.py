@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import cases
-from cases import quad_step
+from cases import LAMBDA0, quad_step
 from genesis4_cuda_port_amd import api
 
 pytestmark = pytest.mark.gpu
@@ -63,3 +63,22 @@ def test_field_copy_is_exact(gpu_ctx, prec):
     assert dst.ring() == (3, 0.25)
     src.close()
     dst.close()
+
+
+@pytest.mark.parametrize("prec", [api.FP64, api.MIXED])
+def test_new_field_is_cleared_before_its_planes_are_set(prec):
+    """A field's planes are zeroed when g4h_field_create returns, so planes set
+    next on any stream stay: each new field, filled at once by a kernel on its
+    context's stream, holds the plane everywhere."""
+    print(f"case field_create_order prec={prec}", flush=True)
+    rng = np.random.default_rng(5)
+    n, g = 64, 129
+    re, im = rng.standard_normal(g * g), rng.standard_normal(g * g)
+    want = (re + 1j * im) if prec == api.FP64 else (re + 1j * im).astype(np.complex64)
+    with api.Context(0) as ctx:
+        for _ in range(4):
+            f = api.Field(ctx, prec, n, g, 0.3e-3, LAMBDA0, LAMBDA0)
+            f.fill_planes(re, im)
+            fr, fi, _ = f.download()
+            assert np.array_equal((fr + 1j * fi).reshape(n, -1), np.broadcast_to(want, (n, g * g)))
+            f.close()
