@@ -14,7 +14,10 @@
 // before it: the host's H makes the product over H segments smaller than
 // 1e-25, two for the usual step lengths, at most 16), and once with that.
 // Recomputing takes the 6 operations per element that a correction by a
-// table of products would take, without the table.
+// table of products would take, without the table.  A value that is not
+// finite does not decay: where a segment's forward run ends with one, all 16
+// segments are chained, so that it reaches the whole line as in a single
+// recurrence.
 //
 // Step A's solution gets step B's explicit part at once, while the row's
 // neighbours are in registers: the x sweep writes (1 + i cs d2x) u*, the y
@@ -113,6 +116,9 @@ __device__ __forceinline__ double2 cfma(double2 a, double2 p, double2 b) {  // a
   return make_double2(fma(p.x, b.x, fma(-p.y, b.y, a.x)), fma(p.x, b.y, fma(p.y, b.x, a.y)));
 }
 
+// Whether v is not finite (or its components add up to no finite number).
+__device__ __forceinline__ bool seg_bad(double2 v) { return !__builtin_isfinite(v.x + v.y); }
+
 // x sweep of rows 16 blk .. of one plane.  tab: the step's table in LDS; buf:
 // the wave's rows of the transpose buffer.  sp: the slice's source inside rc.
 template <class P, int K>
@@ -200,9 +206,10 @@ __device__ __forceinline__ void seg_x(const typename A2<P>::T* u, typename A2<P>
   double2 y = make_double2(0.0, 0.0);
 #pragma unroll
   for (int j = 0; j < K; ++j) y = seg_fwd(tab[j * kSegs + t], v[j], y, cs);
+  const int n = __any(seg_bad(y)) ? kSegs : H;  // segments to chain
   {
     double2 e = y;
-    for (int h = 1; h < H; ++h) e = cfma(y, prod, lane_prev(e));
+    for (int h = 1; h < n; ++h) e = cfma(y, prod, lane_prev(e));
     y = lane_prev(e);
   }
 #pragma unroll
@@ -216,7 +223,7 @@ __device__ __forceinline__ void seg_x(const typename A2<P>::T* u, typename A2<P>
   for (int j = K - 1; j >= 0; --j) w = seg_bwd(tab[j * kSegs + t], v[j], w, cs);
   {
     double2 e = w;
-    for (int h = 1; h < H; ++h) e = cfma(w, prod, lane_next(e));
+    for (int h = 1; h < n; ++h) e = cfma(w, prod, lane_next(e));
     w = lane_next(e);
   }
   double2 right = w;  // u* of the element after this segment
@@ -323,9 +330,13 @@ __device__ __forceinline__ void seg_y(const typename A2<P>::T* in, typename A2<P
 #pragma unroll
   for (int j = 0; j < K; ++j) y = seg_fwd(tab[j * kSegs + t], v[j], y, cs);
   ends[t * kSegLines + c] = y;
+  __shared__ int bad[kSegThreads / kLane];
+  static_assert(kSegThreads / kLane == 4);
+  bad[threadIdx.x / kLane] = __any(seg_bad(y));
   __syncthreads();
+  const int chain = (bad[0] | bad[1] | bad[2] | bad[3]) ? kSegs : H;
   y = make_double2(0.0, 0.0);
-  for (int h = H; h >= 1; --h) {
+  for (int h = chain; h >= 1; --h) {
     const int i = max(t - h, 0);
     const double2 n = cfma(ends[i * kSegLines + c], tab[kSegs * K + i], y);
     y.x = t >= h ? n.x : 0.0;
@@ -344,7 +355,7 @@ __device__ __forceinline__ void seg_y(const typename A2<P>::T* in, typename A2<P
   back[t * kSegLines + c] = w;
   __syncthreads();
   w = make_double2(0.0, 0.0);
-  for (int h = H; h >= 1; --h) {
+  for (int h = chain; h >= 1; --h) {
     const int i = min(t + h, kSegs - 1);
     const double2 n = cfma(back[i * kSegLines + c], tab[kSegs * K + i], w);
     w.x = t + h < kSegs ? n.x : 0.0;

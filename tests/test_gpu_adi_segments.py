@@ -59,3 +59,36 @@ def test_segment_lengths(ngrid, nslice, periods, prec):
     e = relerr(gre + 1j * gim, of.re + 1j * of.im)
     print(f"  r {r:.3g} rel err {e:.3e}", flush=True)
     assert e < dep + 4 * eps * np.sqrt(1 + 16 * r * r)
+
+
+@pytest.mark.parametrize("prec", [api.FP64, api.MIXED])
+@pytest.mark.parametrize("ngrid,bad", [(33, np.nan), (151, np.inf), (255, np.nan), (256, -np.inf)])
+def test_non_finite_values_reach_the_whole_plane(ngrid, bad, prec):
+    """One value that is not finite in a plane: a single recurrence carries it
+    along its row and then along every column, so after one step no cell of
+    the plane is finite, and the planes beside it are untouched (the step's own
+    bound).  Records say so too."""
+    print(f"case segments_non_finite ngrid={ngrid} bad={bad} prec={prec}", flush=True)
+    c = cases.make_case(nslice=3, npart=64, ngrid=ngrid, seed_power=1e6, current=0.0)
+    st = quad_step()
+    plane = ngrid * ngrid
+    re, im = noisy_field(c, scale=0.1)
+    re[plane + (ngrid // 3) * ngrid + ngrid // 2] = bad
+    of = OField(c.nslice, ngrid, c.gridmax, LAMBDA0, c.slicelength, 1, re, im)
+    zero = np.zeros_like(re)
+    _oracle.lib().orc_adi_advance(of.ptr, dp(zero), dp(zero), st.delz)
+    want = (of.re + 1j * of.im).reshape(3, plane)
+    assert not np.isfinite(want[1]).any()
+    with api.Context(0) as ctx:
+        f = gpu_field(ctx, c, prec, kind=api.ADI, re=re, im=im)
+        b = gpu_beam(ctx, c, prec)
+        f.track(b, st, st.delz)
+        gre, gim, _ = f.download()
+        power = f.diag_raw()[:, 0]
+        f.close()
+        b.close()
+    got = (gre + 1j * gim).reshape(3, plane)
+    assert not np.isfinite(got[1]).any()
+    assert list(np.isfinite(power)) == [True, False, True]
+    for p in (0, 2):
+        assert relerr(got[p], want[p]) < (1e-12 if prec == api.FP64 else 1e-6)
