@@ -31,6 +31,8 @@
 // y sweep: 16 columns per workgroup, so its loads and stores are row
 // segments of 16 cells and thread (t, column) holds rows t K .. t K + K
 // without any transpose; the end values cross waves through LDS.
+// Floating-point contraction is off in each function body, as in
+// adi_lines.hpp, so the single-field and the batch kernels round alike.
 // A CU holds three or more workgroups of either, which overlap each other's
 // memory latency.  Times: field_adi.hip, where they are launched.
 #pragma once
@@ -104,15 +106,18 @@ __device__ __forceinline__ double2 lane_next(double2 v) { return row_dpp<0x101>(
 
 // cb (r + i cs y)
 __device__ __forceinline__ double2 seg_fwd(double2 cb, double2 r, double2 y, double cs) {
+#pragma clang fp contract(off)
   const double qx = fma(-cs, y.y, r.x), qy = fma(cs, y.x, r.y);
   return make_double2(fma(cb.x, qx, -(cb.y * qy)), fma(cb.x, qy, cb.y * qx));
 }
 // y + i cs cb u
 __device__ __forceinline__ double2 seg_bwd(double2 cb, double2 y, double2 u, double cs) {
+#pragma clang fp contract(off)
   const double zx = -cs * u.y, zy = cs * u.x;
   return make_double2(fma(cb.x, zx, fma(-cb.y, zy, y.x)), fma(cb.x, zy, fma(cb.y, zx, y.y)));
 }
 __device__ __forceinline__ double2 cfma(double2 a, double2 p, double2 b) {  // a + p b
+#pragma clang fp contract(off)
   return make_double2(fma(p.x, b.x, fma(-p.y, b.y, a.x)), fma(p.x, b.y, fma(p.y, b.x, a.y)));
 }
 
@@ -126,6 +131,7 @@ __device__ __forceinline__ void seg_x(const typename A2<P>::T* u, typename A2<P>
                                       double cs, const double2* tab,
                                       const typename A2<P>::T* sp, int4 rc, int blk,
                                       double* bufs) {
+#pragma clang fp contract(off)
   using T2 = typename A2<P>::T;
   constexpr int E = sizeof(T2);
   constexpr int NI = (kSegs * K + kLane - 1) / kLane;  // row pieces of 64 cells
@@ -294,6 +300,7 @@ __device__ __forceinline__ void seg_y(const typename A2<P>::T* in, typename A2<P
                                       double cs, const double2* tab,
                                       const typename A2<P>::T* sp, int4 rc, int blk,
                                       double2* ends, double* red, double* part, double* centre) {
+#pragma clang fp contract(off)
   using T2 = typename A2<P>::T;
   constexpr int E = sizeof(T2);
   const int c = threadIdx.x % kSegLines, t = threadIdx.x / kSegLines;

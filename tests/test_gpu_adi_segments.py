@@ -92,3 +92,55 @@ def test_non_finite_values_reach_the_whole_plane(ngrid, bad, prec):
     assert list(np.isfinite(power)) == [True, False, True]
     for p in (0, 2):
         assert relerr(got[p], want[p]) < (1e-12 if prec == api.FP64 else 1e-6)
+
+
+def _wave_totals(v):
+    """v [..., 64 lanes] summed as a wave sums it (kernels.hpp wave_total)."""
+    lane = np.arange(64)
+    for perm in (lane ^ 1, lane ^ 2, lane ^ 7, lane ^ 15):  # the last two: mirrored 8 and 16
+        v = v + v[..., perm]
+    return (v[..., 0] + v[..., 16]) + (v[..., 32] + v[..., 48])
+
+
+@pytest.mark.parametrize("ngrid,seg", [(64, 4), (113, 8), (151, 10), (255, 16)])
+def test_field_sums_round_as_written(ngrid, seg):
+    """The y sweep's field sums, bit for bit: every product and sum rounded on
+    its own (no contraction into fused operations), in the order the kernel
+    states: the thread's seg rows from the last to the first, the wave, the
+    four waves, the 16-column blocks."""
+    print(f"case segments_sums ngrid={ngrid}", flush=True)
+    c = cases.make_case(nslice=2, npart=64, ngrid=ngrid, seed_power=1e6, current=0.0, nsteps=1)
+    re, im = noisy_field(c, scale=0.1)
+    with api.Context(0) as ctx:
+        f = gpu_field(ctx, c, api.FP64, kind=api.ADI, re=re, im=im)
+        b = gpu_beam(ctx, c, api.FP64)
+        run = api.Run(ctx, b, f, c.steps, LAMBDA0, c.sample, False, False, 1)
+        run.advance(1)
+        raw = run.download_diag()[1][1]
+        gre, gim, _ = f.download()
+        for x in (run, b, f):
+            x.close()
+    nblk = (ngrid + 15) // 16
+    pad = [np.zeros((2, 16 * seg, 16 * nblk)) for _ in range(2)]
+    for p, a in zip(pad, (gre, gim)):
+        p[:, :ngrid, :ngrid] = a.reshape(2, ngrid, ngrid)
+    # [plane, segment, row, block, column]
+    r, i = (p.reshape(2, 16, seg, nblk, 16) for p in pad)
+    shift = -0.5 * (ngrid - 1)
+    wei = r * r + i * i
+    dy = (np.arange(16 * seg).reshape(1, 16, seg, 1, 1) + shift)
+    terms = [wei, dy * wei, dy * dy * wei, r, i]
+    acc = [np.zeros((2, 16, nblk, 16)) for _ in terms]
+    for j in range(seg - 1, -1, -1):
+        acc = [a + t[:, :, j] for a, t in zip(acc, terms)]
+    sw, s3, s4, s5, s6 = acc
+    dx = (np.arange(16 * nblk).reshape(1, 1, nblk, 16) + shift)
+    for k, a in enumerate((sw, dx * sw, dx * dx * sw, s3, s4, s5, s6)):
+        waves = _wave_totals(a.transpose(0, 2, 1, 3).reshape(2, nblk, 4, 64))
+        tot = np.zeros(2)
+        for blk in range(nblk):
+            part = np.zeros(2)
+            for w in range(4):
+                part = part + waves[:, blk, w]
+            tot = tot + part
+        assert np.array_equal(tot, raw[:, k]), k
