@@ -83,18 +83,19 @@ void device_free(Context* ctx, void* p) {
     (void)hipFree(p);
 }
 
-Context::ParamSlot Context::param_push(const void* data, size_t bytes) {
-  require(bytes <= kParamBytes, "parameter block too large");
-  ParamSlot s;
+Context::ParamRun Context::param_push(const void* data, size_t bytes) {
+  require(bytes <= kParamRun, "parameter block too large");
+  const int n = param_slots(bytes);
+  ParamRun r;
   if (capturing) {
-    require(arena && arena->used < arena->slots, "parameter arena of the capture is full");
+    require(arena && arena->used + n <= arena->slots, "parameter arena of the capture is full");
     char* h = arena->host + static_cast<size_t>(arena->used) * kParamBytes;
     char* d = arena->dev + static_cast<size_t>(arena->used) * kParamBytes;
-    ++arena->used;
+    arena->used += n;
     std::memcpy(h, data, bytes);
     G4_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, stream));
-    s.dev = d;
-    return s;
+    r.dev_ = d;
+    return r;
   }
   if (!param_host) {
     void* h = nullptr;
@@ -106,25 +107,25 @@ Context::ParamSlot Context::param_push(const void* data, size_t bytes) {
     this->bytes += kParamSlots * kParamBytes;
     for (hipEvent_t& e : param_ev) G4_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   }
-  const int k = param_next;
-  param_next = (k + 1) % kParamSlots;
-  if (param_pending[k]) {
-    G4_HIP(hipEventSynchronize(param_ev[k]));
-    param_pending[k] = false;
-  }
+  const int k = param_ring.take(n, [this](int first) { G4_HIP(hipEventSynchronize(param_ev[first])); });
+  if (k < 0) fail(G4H_ERR_DEVICE, "parameter ring: every slot is held by a pass being enqueued");
+  r.ctx_ = this;
+  r.first_ = k;
   char* h = param_host + static_cast<size_t>(k) * kParamBytes;
   char* d = param_dev + static_cast<size_t>(k) * kParamBytes;
   std::memcpy(h, data, bytes);
   G4_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, stream));
-  s.dev = d;
-  s.index = k;
-  return s;
+  r.dev_ = d;
+  return r;
 }
 
-void Context::param_commit(const ParamSlot& s) {
-  if (s.index < 0) return;
-  G4_HIP(hipEventRecord(param_ev[s.index], stream));
-  param_pending[s.index] = true;
+void Context::param_queued(int first) noexcept {
+  if (hipEventRecord(param_ev[first], stream) == hipSuccess) {
+    param_ring.queued(first);
+    return;
+  }
+  (void)hipStreamSynchronize(stream);  // no event: wait for the readers here
+  param_ring.drop(first);
 }
 
 void Context::param_release() {

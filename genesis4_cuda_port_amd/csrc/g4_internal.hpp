@@ -16,9 +16,11 @@
 #include <new>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/g4hip.h"
+#include "slot_ring.hpp"
 
 namespace g4 {
 
@@ -182,22 +184,47 @@ struct Context {
   // Parameter blocks that kernels read through a pointer (rather than as
   // by-value arguments, which the compiler keeps live in scalar registers
   // and spills): staged through pinned host memory into a device ring.
-  // param_push copies one or more blocks into the next slot; param_commit
-  // marks the slot in use until the work enqueued so far on the stream has
-  // run (nothing for an empty slot).
-  static constexpr int kParamSlots = 16;
-  static constexpr size_t kParamBytes = 16384;
-  struct ParamSlot {
-    const void* dev = nullptr;
-    int index = -1;
+  // param_push copies one or more blocks (at most kParamRun bytes) into as
+  // many consecutive slots as they take.  The handle holds them while the
+  // caller enqueues what reads them; from its end, also by an exception, they
+  // are in use until the work enqueued so far has run.  One block of a single
+  // pass takes one slot, so the host runs up to 64 such passes ahead.
+  static constexpr int kParamSlots = 64;
+  static constexpr size_t kParamBytes = 4096;
+  static constexpr size_t kParamRun = 16384;
+  static constexpr int param_slots(size_t bytes) {
+    return static_cast<int>((bytes + kParamBytes - 1) / kParamBytes);
+  }
+  class ParamRun {
+   public:
+    ParamRun() = default;
+    ParamRun(ParamRun&& o) noexcept { swap(o); }
+    ParamRun& operator=(ParamRun&& o) noexcept {
+      swap(o);
+      return *this;
+    }
+    ~ParamRun() {
+      if (ctx_) ctx_->param_queued(first_);
+    }
+    const void* dev() const { return dev_; }
+
+   private:
+    friend struct Context;
+    void swap(ParamRun& o) noexcept {
+      std::swap(ctx_, o.ctx_);
+      std::swap(first_, o.first_);
+      std::swap(dev_, o.dev_);
+    }
+    Context* ctx_ = nullptr;  // null: nothing to give back
+    int first_ = 0;
+    const void* dev_ = nullptr;
   };
   char* param_host = nullptr;
   char* param_dev = nullptr;
-  hipEvent_t param_ev[kParamSlots] = {};
-  bool param_pending[kParamSlots] = {};
-  int param_next = 0;
-  ParamSlot param_push(const void* data, size_t bytes);
-  void param_commit(const ParamSlot& slot);
+  hipEvent_t param_ev[kParamSlots] = {};  // of the run that starts there
+  SlotRing param_ring{kParamSlots};
+  ParamRun param_push(const void* data, size_t bytes);
+  void param_queued(int first) noexcept;
   void param_release();
   // While capturing, blocks go to an arena that lives as long as the graph
   // (a replay reads them again): pinned host and device slots, filled in

@@ -1737,10 +1737,10 @@ void launch_t(Context* ctx, Beam* b, const ParticleParams& p, BeamPtr<P> bp,
   const size_t lds = DEP ? static_cast<size_t>(p.dep.window_cap) * sizeof(double2) : 0;
   const int K = split_of(ctx, b);
   const ParticleParams* tab = how.d_table ? how.d_table : how.d_prm;
-  Context::ParamSlot slot;
+  Context::ParamRun block;
   if (!tab && sizeof(P) == 8) {
-    slot = ctx->param_push(&p, sizeof(p));
-    tab = static_cast<const ParticleParams*>(slot.dev);
+    block = ctx->param_push(&p, sizeof(p));
+    tab = static_cast<const ParticleParams*>(block.dev());
   }
   SplitScratch sp{};
   if (K > 1) {
@@ -1773,7 +1773,6 @@ void launch_t(Context* ctx, Beam* b, const ParticleParams& p, BeamPtr<P> bp,
                          0, ctx->stream, bp, b->off.get(), p, tab, sp, K);
     });
   }
-  ctx->param_commit(slot);
 }
 
 template <class P, int NF, bool DEP, bool TAB>

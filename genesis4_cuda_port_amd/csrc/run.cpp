@@ -114,11 +114,14 @@ struct g4h_run {
   }
 
   // Steps [k0, k1).  Their parameters are planned ahead (the ring moves by
-  // host arithmetic alone) and, in FP64, uploaded as many at a time as a
-  // parameter slot holds: one copy of 4.5 us on the stream per dozen steps
-  // instead of one per step (MIXED passes them by value).
+  // host arithmetic alone) and, in FP64, uploaded as many at a time as one
+  // push takes: one copy of 4.5 us on the stream per dozen steps instead of
+  // one per step (MIXED passes them by value).
+  static constexpr int kChunk = static_cast<int>(Context::kParamRun / sizeof(ParticleParams));
+  // a chunk is held while its steps, with space charge one push each, are enqueued
+  static_assert(kChunk >= 1 &&
+                Context::param_slots(Context::kParamRun) + kChunk < Context::kParamSlots);
   void steps_run(int k0, int k1) {
-    constexpr int kChunk = static_cast<int>(Context::kParamBytes / sizeof(ParticleParams));
     std::vector<Plan> plan;
     std::vector<ParticleParams> blocks;
     while (k0 < k1) {
@@ -141,14 +144,13 @@ struct g4h_run {
         blocks.push_back(q.p);
         if (b->ef.nz > 0) blocks.back().stages &= ~ST_T1;
       }
-      Context::ParamSlot slot;
+      Context::ParamRun held;
       if (b->prec == G4H_FP64)
-        slot = ctx->param_push(blocks.data(), blocks.size() * sizeof(ParticleParams));
-      const auto* dev = static_cast<const ParticleParams*>(slot.dev);
+        held = ctx->param_push(blocks.data(), blocks.size() * sizeof(ParticleParams));
+      const auto* dev = static_cast<const ParticleParams*>(held.dev());
       for (int i = 0; i < n; ++i, ++done)
         step(steps[static_cast<size_t>(k0 + i)], plan[static_cast<size_t>(i)],
              blocks[static_cast<size_t>(i)], dev ? dev + i : nullptr);
-      ctx->param_commit(slot);
       k0 += n;
     }
   }
@@ -288,9 +290,10 @@ g4h_status g4h_run_capture(g4h_run* r) {
   if (r->b->prec == G4H_FP64) {
     // parameter slots: the initial record, the steps' chunks, and with space
     // charge each step's first half
-    constexpr size_t kChunk = Context::kParamBytes / sizeof(ParticleParams);
-    const size_t ns = r->steps.size();
-    const int slots = static_cast<int>(2 + ns / kChunk + (r->b->ef.nz > 0 ? ns : 0));
+    const int ns = static_cast<int>(r->steps.size());
+    auto of = [](int blocks) { return Context::param_slots(blocks * sizeof(ParticleParams)); };
+    const int slots = of(1) + ns / g4h_run::kChunk * of(g4h_run::kChunk) +
+                      of(ns % g4h_run::kChunk) + (r->b->ef.nz > 0 ? ns * of(1) : 0);
     void* h = nullptr;
     void* d = nullptr;
     G4_HIP(hipHostMalloc(&h, static_cast<size_t>(slots) * Context::kParamBytes, hipHostMallocDefault));

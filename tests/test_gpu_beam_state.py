@@ -3,6 +3,8 @@
 (planes and ring state, bit for bit)."""
 from __future__ import annotations
 
+import time
+
 import numpy as np
 import pytest
 
@@ -82,3 +84,35 @@ def test_new_field_is_cleared_before_its_planes_are_set(prec):
             fr, fi, _ = f.download()
             assert np.array_equal((fr + 1j * fi).reshape(n, -1), np.broadcast_to(want, (n, g * g)))
             f.close()
+
+
+def test_fp64_passes_queue_without_the_host_waiting():
+    """60 FP64 passes queued behind about 20 ms of work: each uploads its
+    parameter block through a ring of 64 slots, so none of them waits for the
+    device and the host is done with them long before it."""
+    print("case queue_depth", flush=True)
+    c = cases.make_case(nslice=256, npart=2048, ngrid=101, nsteps=200,
+                        seed_power=1e4)
+    small = cases.make_case(nslice=4, npart=256, ngrid=17)
+    st = quad_step()
+    with api.Context(0) as ctx:
+        work, f = gpu_beam(ctx, c, api.MIXED), gpu_field(ctx, c, api.MIXED)
+        b = gpu_beam(ctx, small, api.FP64)
+        shares = []
+        for _ in range(3):
+            run = api.Run(ctx, work, f, c.steps, LAMBDA0, c.sample, True, False, 1, False)
+            b.track_transverse(st, 1e-3, False)  # the ring's memory, on the first call
+            ctx.synchronize()
+            run.advance(len(c.steps))
+            t0 = time.perf_counter()
+            for k in range(60):
+                b.track_transverse(st, 1e-3, bool(k % 2))
+            t1 = time.perf_counter()
+            ctx.synchronize()
+            t2 = time.perf_counter()
+            shares.append((t1 - t0) / (t2 - t0))
+            run.close()
+        print(f"  host share of the queue's time {shares}", flush=True)
+        for x in (b, work, f):
+            x.close()
+    assert min(shares) < 0.5
