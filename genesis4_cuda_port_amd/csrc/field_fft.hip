@@ -1041,9 +1041,16 @@ bool is_pow2(int g) { return g >= 2 && (g & (g - 1)) == 0; }
 
 // Points Q of the transform pairs that step a line of G points by convolution
 // (sizes below 256 that are not powers of two), else 0.
+// From 17 points Q is at least 64, the smallest with several lanes per line:
+// 32 points on one lane read rows of N cells a lane each and column tiles of
+// 256 columns.  Step with Q = 32 -> 64 (before, two transforms of 64 points):
+//   N = 31, 1024 planes  FP64 95.3 -> 58.6 us (64.5), MIXED 65.7 -> 42.1 (51.2)
+//   N = 17, 1 plane      FP64 30.4 -> 22.0 us (30.3), MIXED 27.4 -> 18.9 (22.9)
+// Up to 16 points one lane per line is as fast or faster (N = 3, 1024 planes:
+// FP64 26.5 us with Q = 4, 39.4 with 64; N = 15: 46.7 with 16, 45.1).
 int half_points(int G) {
   if (G < 3 || G > 256 || is_pow2(G)) return 0;
-  int q = 2;
+  int q = G > 16 ? 64 : 4;
   while (q < G) q *= 2;
   return q;
 }
@@ -1154,7 +1161,6 @@ void with_half(int Q, Fn&& fn) {
     case 4: fn(std::integral_constant<int, 4>{}); break;
     case 8: fn(std::integral_constant<int, 8>{}); break;
     case 16: fn(std::integral_constant<int, 16>{}); break;
-    case 32: fn(std::integral_constant<int, 32>{}); break;
     case 64: fn(std::integral_constant<int, 64>{}); break;
     case 128: fn(std::integral_constant<int, 128>{}); break;
     default: fn(std::integral_constant<int, 256>{}); break;

@@ -1,9 +1,9 @@
 """GPU: spectral line steps by pairs of transforms at the edges of their sizes.
 
 Two deposition + FFT steps against the FP64 oracle at the smallest and largest
-grids of each transform size (64, 128 and 256 points) and at the first grid
-beyond them, for slice counts on both sides of the eight XCDs that the planes
-are dealt to.  The particle pass is split (few slices), so the column pass also
+grids of each transform size (4, 16, 64, 128 and 256 points) and at the first
+grid beyond them, for slice counts on both sides of the eight XCDs that the
+planes are dealt to.  The particle pass is split (few slices), so the column pass also
 clears the source behind itself, which the second step would show.  Bounds of
 the other spectral field-step tests: FP64 1e-12, MIXED 2e-5."""
 from __future__ import annotations
@@ -24,8 +24,8 @@ from test_gpu_parity import gpu_beam, gpu_field, noisy_field, relerr  # noqa: E4
 
 @pytest.mark.parametrize("prec,tol", [(api.FP64, 1e-12), (api.MIXED, 2e-5)])
 @pytest.mark.parametrize("filtered", [False, True])
-@pytest.mark.parametrize("ngrid,nslice", [(33, 9), (63, 8), (65, 1), (127, 3), (129, 9), (255, 2),
-                                          (257, 2)])
+@pytest.mark.parametrize("ngrid,nslice", [(3, 1), (15, 9), (17, 9), (31, 3), (33, 9), (63, 8), (65, 1),
+                                          (127, 3), (129, 9), (255, 2), (257, 2)])
 def test_line_pairs(ngrid, nslice, filtered, prec, tol):
     print(f"case fft lines ngrid={ngrid} nslice={nslice} filter={filtered} prec={prec}", flush=True)
     c = cases.make_case(nslice=nslice, npart=1024, ngrid=ngrid, seed_power=1e6)
