@@ -642,6 +642,12 @@ struct HalfCfg {
   // buffer, so that LDS does not limit the workgroups per CU
   using B = P;
   static constexpr int kMinWaves = S::L == 1 ? 1 : (sizeof(P) == 8 ? 3 : 4);  // per SIMD
+  // The FP64 row pass needs 192 registers: held to the 168 of three waves it
+  // spilled 27 (Q = 128; 16 for 256) and took 239 us on 1024 planes of N = 127,
+  // twice the 124 of two transforms of 256 points.  Step, three -> two waves:
+  // N = 127 376 -> 277 us (362), N = 80 195 -> 177 (186), 256 planes of N = 255
+  // 338 -> 268.
+  static constexpr int kRowWaves = sizeof(P) == 8 ? std::min(kMinWaves, 2) : kMinWaves;
 };
 
 // The step of one line held as v (natural layout): tw the four-step
@@ -691,7 +697,7 @@ __device__ __forceinline__ void half_line_step(T2 (&v)[fftr::Shape<Q>::R], int t
 }
 
 template <class P, int Q>
-__global__ __launch_bounds__((HalfCfg<P, Q>::kThreads), (HalfCfg<P, Q>::kMinWaves)) void
+__global__ __launch_bounds__((HalfCfg<P, Q>::kThreads), (HalfCfg<P, Q>::kRowWaves)) void
 fft_rows_half_kernel(typename C2<P>::T* u, int64_t nrows, int N, const double2* tw_d,
                      const double2* mult_d) {
   using T2 = typename C2<P>::T;
@@ -735,9 +741,7 @@ fft_rows_half_kernel(typename C2<P>::T* u, int64_t nrows, int N, const double2* 
 // XCD (workgroups go to the eight XCDs round robin) and plain accesses:
 // with N odd every row segment cuts cache lines that the neighbouring tiles
 // complete in L2.
-// WORK: the filtered source of the work plane is added (a variant of its own:
-// beside the other source it doubled the registers).
-template <class P, int Q, bool WORK>
+template <class P, int Q>
 __global__ __launch_bounds__((HalfCfg<P, Q>::kThreads), (HalfCfg<P, Q>::kMinWaves)) void
 fft_cols_half_kernel(typename C2<P>::T* u, int nslice, int N, const double2* tw_d,
                      const double2* mult_d, typename C2<P>::T* src, const int4* rect, int first,
@@ -779,9 +783,8 @@ fft_cols_half_kernel(typename C2<P>::T* u, int nslice, int N, const double2* tw_
 
   const int s = ((p - first) % nslice + nslice) % nslice;  // beam slice of this ring plane
   int4 rc = make_int4(0, 0, 0, 0);
-  if (!WORK && add_src == 1) rc = rect[s];
-  const bool src_on =
-      !WORK && add_src == 1 && tile * TW < rc.z && (tile + 1) * TW > rc.x;  // uniform
+  if (add_src == 1) rc = rect[s];
+  const bool src_on = add_src == 1 && tile * TW < rc.z && (tile + 1) * TW > rc.x;  // uniform
   if (src_on) {
     const Rsrc rs = plane_rsrc(src + static_cast<int64_t>(s) * N * N, N, E);
     const bool scol = col >= rc.x && col < rc.z;
@@ -796,11 +799,16 @@ fft_cols_half_kernel(typename C2<P>::T* u, int nslice, int N, const double2* tw_
       if constexpr (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     });
   }
-  if constexpr (WORK) {
+  // The filtered source of the work plane.  Behind a run-time branch, like the
+  // other source: as straight-line code after the line step (a compile-time
+  // variant) it spilled up to 298 registers.
+  if (add_src == 2) {
     const Rsrc rw = plane_rsrc(work + static_cast<int64_t>(p) * N * N, N, 16);
+    uint32_t w0 = cell_off(col < N, t, col, N, 16), wstep = static_cast<uint32_t>(L) * N * 16;
+    asm volatile("" : "+v"(w0), "+s"(wstep));
     fftr::static_for<0, R>([&](auto ic) {
       constexpr int r = decltype(ic)::value;
-      const double2 wv = bload<0, double2>(rw, cell_off(col < N, t + L * r, col, N, 16));
+      const double2 wv = bload<0, double2>(rw, w0 + r * wstep);
       v[r].x += static_cast<P>(wv.x);
       v[r].y += static_cast<P>(wv.y);
       if constexpr (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
@@ -1145,13 +1153,10 @@ void cols_half(Field* f, typename C2<P>::T* data, int add_src, int clear, double
   using C = HalfCfg<P, Q>;
   const int N = f->ngrid;
   const int ntile = (N + C::TW - 1) / C::TW;
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3((f->nslice + 7) / 8 * 8 * ntile), dim3(C::kThreads), 0,
-                       f->ctx->stream, data, f->nslice, N, f->fft_tw_conv.get(), f->fft_prop,
-                       static_cast<T2*>(f->src()), f->src_rect.get(), f->first, add_src, clear,
-                       f->fft_work.get(), partials);
-  };
-  go(add_src == 2 ? fft_cols_half_kernel<P, Q, true> : fft_cols_half_kernel<P, Q, false>);
+  hipLaunchKernelGGL((fft_cols_half_kernel<P, Q>), dim3((f->nslice + 7) / 8 * 8 * ntile),
+                     dim3(C::kThreads), 0, f->ctx->stream, data, f->nslice, N,
+                     f->fft_tw_conv.get(), f->fft_prop, static_cast<T2*>(f->src()),
+                     f->src_rect.get(), f->first, add_src, clear, f->fft_work.get(), partials);
 }
 
 // Calls fn with the compile-time size Q of the transform pairs.
