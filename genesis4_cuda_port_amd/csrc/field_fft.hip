@@ -17,10 +17,11 @@
 //
 // Transforms: power-of-two sizes use register-resident radix-2 transforms
 // (forward DIF, inverse DIT, multipliers in bit-reversed order); other sizes
-// up to 512 step their lines by convolution through such transforms, larger
-// ones and the source filter use a direct DFT in LDS.  With the source filter on (non-separable), the filtered
-// source T = 2 IFFT2(filt FFT2(S))/G^2 is built in a work plane first
-// (FWD rows, FWD*filt*INV columns, INV rows) and added in place of 2S.
+// up to 511 step their lines by convolution through such transforms, larger
+// ones and the source filter use a direct DFT in LDS.  With the source filter
+// on (non-separable), the filtered source T = 2 IFFT2(filt FFT2(S))/G^2 is
+// built in a work plane first (FWD rows, FWD*filt*INV columns, INV rows) and
+// added in place of 2S.
 #include "buffer_access.hpp"
 #include "fft_regs.hpp"
 #include "kernels.hpp"
@@ -610,7 +611,7 @@ __global__ void gather_source_kernel(const typename C2<P>::T* src, const int4* r
 
 // ---------------------------------------------------------------------------
 // Other sizes N < 256 with the propagator: convolution through pairs of
-// Q-point transforms, Q the power of two above N.  One line's step
+// Q-point transforms, Q a power of two above N (half_points).  One line's step
 // IDFT_N(P . DFT_N(u)) is the circular convolution of u with h = IDFT_N(P).
 // With g_k = h_(k mod N), |k| < N, wrapped onto M = 2Q >= 2N - 1 points, a
 // circular convolution of M points gives the line's N values at 0 .. N - 1.
@@ -866,15 +867,17 @@ fft_cols_half_kernel(typename C2<P>::T* u, int nslice, int N, const double2* tw_
 // of O(N^2) per line).
 // ---------------------------------------------------------------------------
 
+constexpr int kConvPoints = 1024;  // M for 257 <= N <= 511
+
 // Launch shape of the convolution passes: as many waves (up to four) as fit
-// their transpose buffers in 72 KiB (48 KiB for MIXED lines of 1024 points,
-// where four waves measured slower than two), the padded lines taking twice
-// the LDS of N-point ones; TW columns per column-pass tile (a power of two).
-template <class P, int M>
+// their transpose buffers in 72 KiB (48 KiB for MIXED, where four waves
+// measured slower than two), the padded lines taking twice the LDS of N-point
+// ones; TW columns per column-pass tile (a power of two).
+template <class P>
 struct ConvCfg {
-  using S = fftr::Shape<M>;
+  using S = fftr::Shape<kConvPoints>;
   static constexpr int kWaveBytes = S::LPW * S::BUF * 2 * static_cast<int>(sizeof(P));
-  static constexpr int kLds = sizeof(P) == 8 || M <= 512 ? 72 * 1024 : 48 * 1024;
+  static constexpr int kLds = sizeof(P) == 8 ? 72 * 1024 : 48 * 1024;
   static constexpr int kWaves = kWaveBytes * 4 <= kLds ? 4 : (kWaveBytes * 2 <= kLds ? 2 : 1);
   static constexpr int kThreads = 64 * kWaves;
   // columns per column-pass tile: one line slot (L lanes) per column
@@ -885,12 +888,13 @@ struct ConvCfg {
 // Row pass: rows of N points, each held on the lanes of a line slot as in
 // fft_rows_reg_kernel (without its prefetch: the padded lines already take
 // twice the registers).
-template <class P, int M>
-__global__ __launch_bounds__((ConvCfg<P, M>::kThreads)) void fft_rows_conv_kernel(
+template <class P>
+__global__ __launch_bounds__((ConvCfg<P>::kThreads)) void fft_rows_conv_kernel(
     typename C2<P>::T* u, int64_t nrows, int N, const double2* tw_d, const double2* mult_d) {
   using T2 = typename C2<P>::T;
+  constexpr int M = kConvPoints;
   using S = fftr::Shape<M>;
-  using C = ConvCfg<P, M>;
+  using C = ConvCfg<P>;
   constexpr int R = S::R, L = S::L;
   __shared__ T2 tw[M];
   __shared__ T2 mu[M];
@@ -939,14 +943,15 @@ __global__ __launch_bounds__((ConvCfg<P, M>::kThreads)) void fft_rows_conv_kerne
 // written back with 2S added inside the slice's source rectangle (or the
 // filtered source of the work plane) and the field sums of the tile.
 
-template <class P, int M>
-__global__ __launch_bounds__((ConvCfg<P, M>::kThreads)) void fft_cols_conv_kernel(
+template <class P>
+__global__ __launch_bounds__((ConvCfg<P>::kThreads)) void fft_cols_conv_kernel(
     typename C2<P>::T* u, int nslice, int N, const double2* tw_d, const double2* mult_d,
     typename C2<P>::T* src, const int4* rect, int first, int add_src, int clear_src,
     const double2* work, double* partials) {
   using T2 = typename C2<P>::T;
+  constexpr int M = kConvPoints;
   using S = fftr::Shape<M>;
-  using C = ConvCfg<P, M>;
+  using C = ConvCfg<P>;
   constexpr int R = S::R, L = S::L, TW = C::TW;
   static_assert(C::kThreads / TW == L, "one line slot per column, L lanes each");
   __shared__ T2 tw[M];
@@ -1064,7 +1069,7 @@ int half_points(int G) {
 }
 // Points M of the transforms that step larger lines by convolution (257 to
 // 511), else 0.
-int conv_points(int G) { return G > 256 && G < 512 ? 1024 : 0; }
+int conv_points(int G) { return G > 256 && G < 512 ? kConvPoints : 0; }
 
 // Launch shape of the DFT kernels (sizes that are not powers of two).
 struct DftCfg {
@@ -1109,26 +1114,26 @@ void cols_reg(Field* f, typename C2<P>::T* data, int mode, double scale, int add
                      f->src_rect.get(), f->first, add_src, clear, f->fft_work.get(), partials);
 }
 
-template <class P, int M>
+template <class P>
 void rows_conv(Field* f, typename C2<P>::T* data) {
-  using C = ConvCfg<P, M>;
-  constexpr int LPW = fftr::Shape<M>::LPW;
+  using C = ConvCfg<P>;
+  constexpr int LPW = C::S::LPW;
   const int N = f->ngrid;
   const int64_t nrows = static_cast<int64_t>(f->nslice) * N;
   const int64_t ngroups = (nrows + LPW - 1) / LPW;
   const int64_t nblk = std::min<int64_t>((ngroups + C::kWaves - 1) / C::kWaves, 8192);
-  hipLaunchKernelGGL((fft_rows_conv_kernel<P, M>), dim3(static_cast<unsigned>(nblk)),
+  hipLaunchKernelGGL((fft_rows_conv_kernel<P>), dim3(static_cast<unsigned>(nblk)),
                      dim3(C::kThreads), 0, f->ctx->stream, data, nrows, N, f->fft_tw_conv.get(),
                      f->fft_prop);
 }
 
-template <class P, int M>
+template <class P>
 void cols_conv(Field* f, typename C2<P>::T* data, int add_src, int clear, double* partials) {
   using T2 = typename C2<P>::T;
-  using C = ConvCfg<P, M>;
+  using C = ConvCfg<P>;
   const int N = f->ngrid;
-  const int ntile = (N + ConvCfg<P, M>::TW - 1) / ConvCfg<P, M>::TW;
-  hipLaunchKernelGGL((fft_cols_conv_kernel<P, M>), dim3(f->nslice * ntile), dim3(C::kThreads), 0,
+  const int ntile = (N + C::TW - 1) / C::TW;
+  hipLaunchKernelGGL((fft_cols_conv_kernel<P>), dim3(f->nslice * ntile), dim3(C::kThreads), 0,
                      f->ctx->stream, data, f->nslice, N, f->fft_tw_conv.get(), f->fft_prop,
                      static_cast<T2*>(f->src()), f->src_rect.get(), f->first, add_src, clear,
                      f->fft_work.get(), partials);
@@ -1201,7 +1206,7 @@ int col_tile(int G, size_t esz) {
     return tc;
   }
   if (conv_points(G))
-    return esz == sizeof(double2) ? ConvCfg<double, 1024>::TW : ConvCfg<float, 1024>::TW;
+    return esz == sizeof(double2) ? ConvCfg<double>::TW : ConvCfg<float>::TW;
   if (!is_pow2(G)) return dft_cfg(G, esz).tc;
   int tc = 0;
   with_pow2(G, [&](auto g) {
@@ -1225,7 +1230,7 @@ void run_rows(Field* f, typename C2<P>::T* data, int mode, double scale) {
       return;
     }
     if (mode == ROW_PROP && conv_points(G)) {
-      rows_conv<P, 1024>(f, data);
+      rows_conv<P>(f, data);
       return;
     }
     const DftCfg c = dft_cfg(G, sizeof(T2));
@@ -1261,7 +1266,7 @@ void run_cols(Field* f, typename C2<P>::T* data, int mode, double scale, int add
       return;
     }
     if (mode == COL_PROP && conv_points(G)) {
-      cols_conv<P, 1024>(f, data, add_src, clr, partials);
+      cols_conv<P>(f, data, add_src, clr, partials);
       return;
     }
     const DftCfg c = dft_cfg(G, sizeof(T2));

@@ -1254,7 +1254,7 @@ __device__ __forceinline__ void particle_slice(BeamPtr<P> b, const int32_t* off,
 
   const int tid = threadIdx.x;
   // With K > 1 the slice's particles are split into K contiguous parts, one
-  // per workgroup; the last part to finish combines them.
+  // per workgroup; a following launch combines them.
   const int64_t i0s = off[s], i1s = off[s + 1];
   int64_t i0 = i0s, i1 = i1s;
   if (K > 1) {
@@ -1929,7 +1929,7 @@ __global__ __launch_bounds__(kThreads) void batch_step_particle_kernel(
 // split run (one workgroup each), the slice's source rectangle and footprint
 // from the boxes its parts folded with atomics (then emptied for the next
 // step) and, with sums, the slice's beam sums from the K parts' partial sums
-// in part order: what the last part of a counting launch does.
+// in part order.
 template <class P>
 __global__ __launch_bounds__(256) void batch_publish_kernel(const BatchRunDesc* __restrict__ runs,
                                                             int k, int sums) {
@@ -2137,8 +2137,8 @@ void launch_batch_step_particles(Context* ctx, g4h_precision prec, int nharm,
 // ---- beam sums without allocation ----------------------------------------
 // Device memory for callers that cannot allocate (code under graph capture,
 // tight serving loops): the FP64 parameter block, the per-slice sums before
-// their copy to the host, and the split pass's per-part partials and
-// per-slice arrival counters all live in this array.  Each GPU the library
+// their copy to the host, and the split pass's per-part partials and boxes
+// all live in this array.  Each GPU the library
 // runs on holds its own copy until the process ends.  Host code must use the
 // address from hipGetSymbolAddress (scratch_base), never the array's name.
 static __device__ __align__(256) double scratch[kNoallocScratchBytes / sizeof(double)];

@@ -99,6 +99,16 @@ def test_inverse_normal_matches_ndtri():
     assert np.max(np.abs(ours - ref) / np.maximum(1, np.abs(ref))) < 1e-14
 
 
+def test_inverse_normal_in_the_far_tails():
+    """Down to half a step of a 32-bit point, where the iteration's start is off
+    by up to 1.6 and takes up to 8 steps: the value to rounding, both tails."""
+    tail = np.concatenate([0.5 / 2.0 ** 32 * np.arange(1, 40, 2), np.geomspace(1e-9, 1e-2, 200)])
+    for p in (tail, 1.0 - tail):
+        ours = np.array([api.inverse_normal(v) for v in p])
+        ref = np.where(p > 0.5, -special.ndtri(1.0 - p), special.ndtri(p))
+        assert np.max(np.abs(ours - ref) / np.abs(ref)) < 1e-14
+
+
 def test_lattice_fodo_table():
     steps = api.lattice_fodo(0.026, [1.7, 1.6], 50, 46, 3, 1.5, 2)
     assert len(steps) == 100

@@ -254,8 +254,9 @@ def test_field_track_fp64(gpu_ctx, kind, ngrid):
 def test_fft_sizes(gpu_ctx, prec, ngrid):
     """Spectral step at every transform shape: one or several lines per wave
     (G < 64), one to sixteen points per lane (G >= 64); sizes that are not
-    powers of two up to 512 through the convolution by M-point transforms
-    (M = 8 ... 1024), larger ones (600) through the direct DFT."""
+    powers of two through pairs of transforms (below 256: 4 ... 16 and 64 ... 256
+    points), through transforms of 1024 points (to 511), larger ones (600)
+    through the direct DFT."""
     print(f"case fft_sizes prec={prec} ngrid={ngrid}", flush=True)
     ns = 1 if ngrid == 600 else 3  # the oracle's direct DFT at 600 takes seconds per plane
     first = 2 % ns

@@ -2,7 +2,7 @@
 
 The three single-chain ADI variants (workgroup per plane; wave per 64 lines
 with 8- or 16-element load chunks) must give bit-identical fields and field
-sums; each of them and the segmented variant 3 (16 waves per 64 lines, every
+sums; each of them and the segmented variant 3 (16 lanes per line, every
 element in registers) must match the FP64 oracle with the source on; the
 lane variants must cover grids the workgroup variant cannot hold in LDS
 (G > 360); an unpinned context runs the segmented sweeps for G <= 256
