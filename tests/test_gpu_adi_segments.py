@@ -1,16 +1,18 @@
 """GPU: segmented ADI sweeps at the edges of their segment lengths.
 
-One field step with the source on against the FP64 oracle at the smallest and
+Two field steps with the source on against the FP64 oracle at the smallest and
 largest grid of every segment length (4, 7, 8, 10, 13 and 16 elements on 16
 lanes), for slice counts on both sides of the eight XCDs the planes are dealt
 to, and for step lengths from one undulator period to 3000 (coefficient r from
 below 0.1 to above 10, where a line couples over all its segments instead of
-two).  Both sides solve (1 - i r d2) twice; its condition number is
-sqrt(1 + 16 r^2) and a solve rounds within about G eps of it, so the fields
-agree within 4 G eps sqrt(1 + 16 r^2) (MIXED: the field is rounded to FP32
-after each sweep, 4 sqrt(1 + 16 r^2) 2^-24), plus the deposition's own error:
-1e-13 for the order of its FP64 sums, 2e-5 for MIXED's FP32 terms, the bound
-of the other field-step tests."""
+two).  The particle pass is split, so the y sweep also clears the source
+behind itself, which the second step would show.  Both sides solve (1 - i r d2)
+twice a step; its condition number is sqrt(1 + 16 r^2) and a solve rounds
+within about G eps of it, so the fields agree within 4 G eps sqrt(1 + 16 r^2)
+a step (MIXED: the field is rounded to FP32 after each sweep, 4 sqrt(1 + 16
+r^2) 2^-24), plus the deposition's own error: 1e-13 for the order of its FP64
+sums, 2e-5 for MIXED's FP32 terms, the bound of the other field-step tests.
+The field records of a run at the same grids cover the sweep with sums."""
 from __future__ import annotations
 
 import numpy as np
@@ -34,31 +36,65 @@ from test_gpu_parity import gpu_beam, gpu_field, noisy_field, relerr  # noqa: E4
                                           (209, 1), (256, 3)])
 def test_segment_lengths(ngrid, nslice, periods, prec):
     print(f"case segments ngrid={ngrid} nslice={nslice} periods={periods} prec={prec}", flush=True)
-    c = cases.make_case(nslice=nslice, npart=256, ngrid=ngrid, seed_power=1e6)
+    c = cases.make_case(nslice=nslice, npart=1024, ngrid=ngrid, seed_power=1e6)
     st = quad_step()
     delz = st.delz * periods
     first = nslice // 2
     re, im = noisy_field(c, scale=0.1)
     of = OField(c.nslice, c.ngrid, c.gridmax, LAMBDA0, c.slicelength, 1, re, im, first=first)
     o = c.beam
-    sre = np.zeros(c.nslice * ngrid * ngrid)
-    sim = np.zeros_like(sre)
+    r = 0.25 * delz / (2 * np.pi / LAMBDA0 * (2 * c.gridmax / (ngrid - 1)) ** 2)
+    eps, dep = (ngrid * 2.0 ** -53, 1e-13) if prec == api.FP64 else (2.0 ** -24, 2e-5)
     with api.Context(0) as ctx:
         f = gpu_field(ctx, c, prec, kind=api.ADI, re=re, im=im, first=first)
         b = gpu_beam(ctx, c, prec)
-        f.track(b, st, delz)
-        gre, gim, _ = f.download()
+        for n in (1, 2):
+            f.track(b, st, delz)
+            sre = np.zeros(c.nslice * ngrid * ngrid)
+            sim = np.zeros_like(sre)
+            assert _oracle.lib().orc_deposit(c.nslice, ip(o.offsets), dp(o.x), dp(o.y),
+                                             dp(o.gamma), dp(o.theta), of.ptr, st, dp(o.current),
+                                             delz, dp(sre), dp(sim)) == 1
+            _oracle.lib().orc_adi_advance(of.ptr, dp(sre), dp(sim), delz)
+            gre, gim, _ = f.download()
+            e = relerr(gre + 1j * gim, of.re + 1j * of.im)
+            print(f"  step {n} r {r:.3g} rel err {e:.3e}", flush=True)
+            assert e < dep + n * 4 * eps * np.sqrt(1 + 16 * r * r)
         f.close()
         b.close()
-    assert _oracle.lib().orc_deposit(c.nslice, ip(o.offsets), dp(o.x), dp(o.y), dp(o.gamma),
-                                     dp(o.theta), of.ptr, st, dp(o.current), delz, dp(sre),
-                                     dp(sim)) == 1
-    _oracle.lib().orc_adi_advance(of.ptr, dp(sre), dp(sim), delz)
-    r = 0.25 * delz / (2 * np.pi / LAMBDA0 * (2 * c.gridmax / (ngrid - 1)) ** 2)
-    eps, dep = (ngrid * 2.0 ** -53, 1e-13) if prec == api.FP64 else (2.0 ** -24, 2e-5)
-    e = relerr(gre + 1j * gim, of.re + 1j * of.im)
-    print(f"  r {r:.3g} rel err {e:.3e}", flush=True)
-    assert e < dep + 4 * eps * np.sqrt(1 + 16 * r * r)
+
+
+@pytest.mark.parametrize("prec", [api.FP64, api.MIXED])
+@pytest.mark.parametrize("ngrid,nslice", [(3, 1), (64, 3), (65, 8), (112, 2), (113, 3), (128, 9),
+                                          (129, 1), (160, 2), (161, 3), (208, 2), (209, 1),
+                                          (256, 3)])
+def test_segment_length_records(ngrid, nslice, prec):
+    """Field records of a three-step run (sums, centre cell, slippage) against
+    the oracle's run: each sum within the run tests' bounds (FP64 1e-10, MIXED
+    1e-3) of the power times the moment's weight at the grid's edge."""
+    print(f"case segment_records ngrid={ngrid} nslice={nslice} prec={prec}", flush=True)
+    c = cases.make_case(nslice=nslice, npart=1024, ngrid=ngrid, nsteps=3, seed_power=1e6)
+    re, im = noisy_field(c, scale=0.1)
+    of = OField(c.nslice, ngrid, c.gridmax, LAMBDA0, c.slicelength, 1, re, im)
+    _, _, want = _oracle.run(c.beam, of, c.steps, gamma0=cases.GAMMA0, lambda0=LAMBDA0,
+                             solver=api.ADI, sample=c.sample, timerun=c.timerun)
+    with api.Context(0) as ctx:
+        f = gpu_field(ctx, c, prec, kind=api.ADI, re=re, im=im)
+        b = gpu_beam(ctx, c, prec)
+        run = api.Run(ctx, b, f, c.steps, LAMBDA0, c.sample, c.timerun, False, 1)
+        run.advance(3)
+        got = run.download_diag()[1]
+        for x in (run, b, f):
+            x.close()
+    assert got.shape == want.shape
+    power = want[:, :, 0].max()
+    h = 0.5 * (ngrid - 1)
+    amp = np.sqrt(power)
+    scale = np.array([power, power * h, power * h * h, power * h, power * h * h, amp * ngrid,
+                      amp * ngrid, amp, amp])
+    e = np.abs(got - want).max(axis=(0, 1)) / scale
+    print(f"  rel err {np.array2string(e, precision=1)}", flush=True)
+    assert (e < (1e-10 if prec == api.FP64 else 1e-3)).all()
 
 
 @pytest.mark.parametrize("prec", [api.FP64, api.MIXED])
