@@ -961,16 +961,17 @@ struct SplitScratch {
 };
 
 // Folds the cells that particles [i0, i1) touch into LDS box[0..3] (min x,
-// min y, max x, max y; set empty before); valid after the next barrier.
-template <class P>
+// min y, max x, max y; set empty before), by NT threads; valid after the next
+// barrier.
+template <int NT, class P>
 __device__ __forceinline__ void fold_footprint(BeamPtr<P> b, int64_t i0, int64_t i1,
-                                               const DepParams& d, int* box) {
+                                               const ParticleParams& prm, int ng, int* box) {
   int mnx = 0x7fffffff, mny = 0x7fffffff, mxx = -1, mxy = -1;
-  for (int64_t k = i0 + threadIdx.x; k < i1; k += blockDim.x) {
+  for (int64_t k = i0 + threadIdx.x; k < i1; k += NT) {
     int ix, iy;
     P wx, wy;
-    if (cell_of<P>(b.x[k], b.y[k], P(d.gridmax), P(d.dgrid), P(d.inv_dgrid), d.ngrid, ix, iy, wx,
-                   wy)) {
+    if (cell_of<P>(b.x[k], b.y[k], P(prm.dep.gridmax), P(prm.dep.dgrid), P(prm.dep.inv_dgrid), ng,
+                   ix, iy, wx, wy)) {
       mnx = min(mnx, ix);
       mny = min(mny, iy);
       mxx = max(mxx, ix + 1);
@@ -1286,7 +1287,7 @@ __device__ __forceinline__ void particle_slice(BeamPtr<P> b, const int32_t* off,
         s_bb[2] = s_bb[3] = -1;
       }
       __syncthreads();
-      fold_footprint(b, i0s, i1s, prm.dep, s_bb);
+      fold_footprint<NT>(b, i0s, i1s, prm, ng, s_bb);
       __syncthreads();
       bb = make_int4(s_bb[0], s_bb[1], s_bb[2], s_bb[3]);
       __syncthreads();
@@ -1602,7 +1603,7 @@ __global__ __launch_bounds__(kThreads) void split_combine_kernel(
     // through the global atomics.  The positions after this pass give it.
     __syncthreads();
     if (s_none && prm.dep.cur_over_npar[s] != 0.0) {
-      fold_footprint(b, off[s], off[s + 1], prm.dep, s_bb);
+      fold_footprint<kThreads>(b, off[s], off[s + 1], prm, prm.dep.ngrid, s_bb);
       __syncthreads();
       if (tid == 0 && s_bb[0] <= s_bb[2])
         prm.dep.bbox[s] = make_int4(s_bb[0], s_bb[1], s_bb[2], s_bb[3]);
@@ -1689,7 +1690,7 @@ __global__ void split_prepass_kernel(BeamPtr<P> b, const int32_t* off, ParticleP
     s_bb[2] = s_bb[3] = -1;
   }
   __syncthreads();
-  fold_footprint(b, off[s], off[s + 1], prm.dep, s_bb);
+  fold_footprint<kThreads>(b, off[s], off[s + 1], prm, prm.dep.ngrid, s_bb);
   __syncthreads();
   // stays empty when no particle is on the grid: every part then deposits
   // through the global fallback
@@ -1757,7 +1758,7 @@ void launch_t(Context* ctx, Beam* b, const ParticleParams& p, BeamPtr<P> bp,
     sp.wb = sp.tb + parts;
     if (DEP && how.prepass) {
       ctx->launch(G4H_K_OTHER, [&] {
-        hipLaunchKernelGGL((split_prepass_kernel<P, TAB>), dim3(b->nslice), dim3(256), 0,
+        hipLaunchKernelGGL((split_prepass_kernel<P, TAB>), dim3(b->nslice), dim3(kThreads), 0,
                            ctx->stream, bp, b->off.get(), p, tab);
       });
     }
