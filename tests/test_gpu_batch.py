@@ -146,3 +146,37 @@ def test_batch_launch_modes_agree(prec):
                   flush=True)
             assert ep < tol and eb < tol, (v, i)
             assert np.array_equal(b0[:, 12], b1[:, 12])  # particle counts
+
+
+@pytest.mark.parametrize("prec", [api.FP64, api.MIXED])
+def test_batch_field_records_equal_lone_runs(gpu_ctx, prec):
+    """Every number of the field records of 40 runs (more than a workgroup of
+    the record kernel takes) on grids of 3 and 9 line blocks.  No current, so
+    no deposition: equal bit for bit to lone runs, whose sweeps and sums take
+    the same order."""
+    print(f"case batch field records prec={prec}", flush=True)
+    steps = _steps()
+    runs = [dict(npart=64, nbins=4, ngrid=(33, 129)[i % 2], gridmax=GRIDMAX, current=0.0,
+                 gamma0=GAMMA0, espread_rel=1e-4, seed=1 + i, seed_power=1e4 * (1 + i),
+                 seed_w0=40e-6) for i in range(40)]
+    batch = api.Batch(gpu_ctx, prec, api.ADI, runs, steps, LAMBDA0)
+    assert batch.advance(NSTEPS) == NSTEPS
+    for i in (0, 1, 15, 30, 33, 38, 39):
+        r = runs[i]
+        _, fraw = batch.download(i)
+        g = r["ngrid"]
+        re, im = api.seed_gaussian(1, g, GRIDMAX, LAMBDA0, r["seed_power"], r["seed_w0"])
+        b = api.Beam(gpu_ctx, prec, np.array([0, 64]), np.zeros(1), GAMMA0)
+        z = np.zeros(64)
+        b.upload(z, z, z, z, np.full(64, GAMMA0), z)
+        f = api.Field(gpu_ctx, prec, 1, g, GRIDMAX, LAMBDA0, LAMBDA0)
+        f.upload(re, im, 0)
+        f.init_solver(api.ADI)
+        run = api.Run(gpu_ctx, b, f, steps, LAMBDA0, 1.0, False, False, 1)
+        run.advance(NSTEPS)
+        want = run.download_diag()[1][:, 0]
+        assert want[:, 0].min() > 0
+        assert np.array_equal(fraw, want), i
+        for x in (run, f, b):
+            x.close()
+    batch.close()
