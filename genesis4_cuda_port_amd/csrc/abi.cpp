@@ -627,6 +627,8 @@ g4h_status g4h_field_create(g4h_context* ctx, g4h_precision precision, int nslic
     f->xks = 4. * std::asin(1) / f->xlambda;                  // Field.cpp:80
     f->slicelength = slicelength;
     const size_t cells = static_cast<size_t>(f->cells());
+    // cleared on the context's stream, ahead of whatever sets planes there next;
+    // blocking copies wait for that stream first
     if (precision == G4H_FP64) {
       f->ud.alloc(ctx, cells);
       G4_HIP(hipMemsetAsync(f->ud.get(), 0, cells * sizeof(double2), ctx->stream));
@@ -634,9 +636,6 @@ g4h_status g4h_field_create(g4h_context* ctx, g4h_precision precision, int nslic
       f->uf.alloc(ctx, cells);
       G4_HIP(hipMemsetAsync(f->uf.get(), 0, cells * sizeof(float2), ctx->stream));
     }
-    // cleared before anyone writes planes, on this stream, another one (another
-    // context's work) or by a blocking copy
-    G4_HIP(hipStreamSynchronize(ctx->stream));
   } catch (...) {
     delete f;
     throw;

@@ -623,12 +623,12 @@ __global__ void gather_source_kernel(const typename C2<P>::T* src, const int4* r
 // M-point ones whose upper half is zeros on the way in and dropped on the way
 // out.  Registers hold two Q-point lines, the transpose buffers one.
 // Bound: VALU and LDS (four 256-point transforms where a power-of-two line has
-// two); the FP64 column pass reaches 4.0 TB/s.  Addresses are 32-bit buffer
-// offsets: 64-bit ones, live from the loads to the stores, took 205 registers
-// where the MIXED passes now take 88 and 115.  Column + row pass, two M-point
-// transforms -> this:
+// two); at N = 255 the FP64 passes move their bytes at 4.4 and 3.9 TB/s.
+// Addresses are 32-bit buffer offsets: 64-bit ones, live from the loads to the
+// stores, took 205 registers where the MIXED passes now take 90 and 115.
+// Column + row pass, two M-point transforms -> this:
 //   1024 planes, N = 151, MIXED   257 + 187 us -> 162 + 142 us
-//   256 planes, N = 255, FP64     495 + 348 us -> 134 + 209 us
+//   256 planes, N = 255, FP64     495 + 348 us -> 137 + 141 us
 // N from 257 (two lines of 512 points, 256 registers in FP64) stays with the
 // M-point transforms below.
 // ---------------------------------------------------------------------------

@@ -69,9 +69,9 @@ def test_field_copy_is_exact(gpu_ctx, prec):
 
 @pytest.mark.parametrize("prec", [api.FP64, api.MIXED])
 def test_new_field_is_cleared_before_its_planes_are_set(prec):
-    """A field's planes are zeroed when g4h_field_create returns, so planes set
-    next on any stream stay: each new field, filled at once by a kernel on its
-    context's stream, holds the plane everywhere."""
+    """A field's planes are zeroed on its context's stream, so planes set next
+    stay: each new field, filled at once by a kernel on that stream, holds the
+    plane everywhere."""
     print(f"case field_create_order prec={prec}", flush=True)
     rng = np.random.default_rng(5)
     n, g = 64, 129
