@@ -124,6 +124,11 @@ __device__ __forceinline__ double2 cfma(double2 a, double2 p, double2 b) {  // a
 // Whether v is not finite (or its components add up to no finite number).
 __device__ __forceinline__ bool seg_bad(double2 v) { return !__builtin_isfinite(v.x + v.y); }
 
+// H of the table, as a scalar (the loops over it are uniform).
+__device__ __forceinline__ int seg_chain(const double2* tab, int K) {
+  return __builtin_amdgcn_readfirstlane(static_cast<int>(tab[kSegs * K + kSegs].x));
+}
+
 // x sweep of rows 16 blk .. of one plane.  tab: the step's table in LDS; buf:
 // the wave's rows of the transpose buffer.  sp: the slice's source inside rc.
 template <class P, int K>
@@ -141,7 +146,7 @@ __device__ __forceinline__ void seg_x(const typename A2<P>::T* u, typename A2<P>
   if (row0 >= G) return;
   const int g = lane / kSegs, t = lane % kSegs;
   double* buf = bufs + 4 * wave * RP;
-  const int H = static_cast<int>(tab[kSegs * K + kSegs].x);
+  const int H = seg_chain(tab, K);
   const Rsrc ru = plane_rsrc(u, G, E);
   const Rsrc ro = plane_rsrc(out, G, E);
   const Rsrc rs = plane_rsrc(sp, G, E);
@@ -306,7 +311,7 @@ __device__ __forceinline__ void seg_y(const typename A2<P>::T* in, typename A2<P
   const int c = threadIdx.x % kSegLines, t = threadIdx.x / kSegLines;
   const int col = blk * kSegLines + c;
   const int row0 = t * K;
-  const int H = static_cast<int>(tab[kSegs * K + kSegs].x);
+  const int H = seg_chain(tab, K);
   const Rsrc ri = plane_rsrc(in, G, E);
   const Rsrc ro = plane_rsrc(u, G, E);
   const Rsrc rs = plane_rsrc(sp, G, E);
@@ -337,11 +342,12 @@ __device__ __forceinline__ void seg_y(const typename A2<P>::T* in, typename A2<P
 #pragma unroll
   for (int j = 0; j < K; ++j) y = seg_fwd(tab[j * kSegs + t], v[j], y, cs);
   ends[t * kSegLines + c] = y;
-  __shared__ int bad[kSegThreads / kLane];
   static_assert(kSegThreads / kLane == 4);
-  bad[threadIdx.x / kLane] = __any(seg_bad(y));
+  __shared__ int4 bad;
+  reinterpret_cast<int*>(&bad)[threadIdx.x / kLane] = __any(seg_bad(y));
   __syncthreads();
-  const int chain = (bad[0] | bad[1] | bad[2] | bad[3]) ? kSegs : H;
+  const int4 nf = bad;
+  const int chain = __builtin_amdgcn_readfirstlane(nf.x | nf.y | nf.z | nf.w) ? kSegs : H;
   y = make_double2(0.0, 0.0);
   for (int h = chain; h >= 1; --h) {
     const int i = max(t - h, 0);
