@@ -2138,8 +2138,9 @@ void launch_batch_step_particles(Context* ctx, g4h_precision prec, int nharm,
 // ---- beam sums without allocation ----------------------------------------
 // Device memory for callers that cannot allocate (code under graph capture,
 // tight serving loops): the FP64 parameter block, the per-slice sums before
-// their copy to the host, and the split pass's per-part partials and boxes
-// all live in this array.  Each GPU the library
+// their copy to the host, and the split pass's per-part partials all live in
+// this array (beam sums do not write the room for the parts' boxes, which
+// counts towards the limit).  Each GPU the library
 // runs on holds its own copy until the process ends.  Host code must use the
 // address from hipGetSymbolAddress (scratch_base), never the array's name.
 static __device__ __align__(256) double scratch[kNoallocScratchBytes / sizeof(double)];
